@@ -117,8 +117,9 @@ enum {
     QS_PATH_GREEDY = 0,  /* temperature <= 0: argmax, no draw */
     QS_PATH_FAST = 1,    /* exact softmax denominator, top candidates preselected by logit,
                             exact order proven */
-    QS_PATH_FULL = 2,    /* whole window sorted on the device (large nucleus, ties across
-                            the preselection boundary, non-finite maxima) */
+    QS_PATH_FULL = 2,    /* decided over the whole window on the device, by selection or by
+                            sorting it (large nucleus, ties across the preselection
+                            boundary, non-finite maxima) */
     QS_PATH_EMPTY = 3,   /* empty window (temperature NaN or 1/T overflowing on a zero
                             max): id 0, as documented in quasar_sampler_pick */
     QS_PATH_CERT = 4     /* the streaming kernel's path: the denominator bounded to an

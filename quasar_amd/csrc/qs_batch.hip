@@ -635,6 +635,11 @@ struct qs_batch {
     uint32_t *d_hbits = nullptr;           // its history bitmap (zero between picks)
     bool hbits_dirty = false;              // a fused pick failed after marking it: clear
                                            // it before the next one
+    OpenScratch open{};                    // rows without a top-k (allocated when one is
+                                           // configured)
+    void *d_open = nullptr;                // its one allocation
+    bool open_dirty = false;               // a launch failed between its two kernels: its
+                                           // counters are cleared before the next pick
     int32_t *h_pin = nullptr;              // pinned: a one-row pick's id and error flag
     int32_t *d_pin = nullptr;              // the device's address of h_pin
 };
@@ -647,7 +652,7 @@ static void batch_release(qs_batch *b) {
                     b->sc.crej, b->sc.cflag, b->sc.psum, b->sc.pcnt, b->sc.locks,
                     b->sc.full_keys, b->sc.full_bm, b->sc.err, b->sc.wrec,
                     b->sc.pcand, b->sc.gbest, b->sc.gmaxk, b->sc.gcnt, b->d_hrec,
-                    b->d_hbits};
+                    b->d_hbits, b->d_open};
     for (void *p : ptrs)
         if (p) (void)hipFree(p);
     if (b->h_pin) (void)hipHostFree(b->h_pin);
@@ -715,6 +720,34 @@ static int batch_alloc(qs_batch *b) {
     if (!rc && hipMemset(b->sc.gmaxk, 0, sizeof(uint32_t) * R) != hipSuccess) rc = QS_EDEVICE;
     if (!rc && hipMemset(b->sc.gcnt, 0, sizeof(uint32_t) * R) != hipSuccess) rc = QS_EDEVICE;
     return rc;
+}
+
+// Scratch of the whole-window decision for rows without a top-k (qs_open.h), for the first
+// QS_OPEN_ROWS rows of a pick: one allocation, zeroed once (each pick leaves hist, cnt and
+// done zero).  Without it such rows decide in their own workgroup, so no room is no error.
+static void open_alloc(qs_batch *b) {
+    if (b->d_open || qs_part_parts(b->max_vocab) > QS_PART_MAX_PARTS) return;
+    const size_t R = b->max_rows < QS_OPEN_ROWS ? b->max_rows : QS_OPEN_ROWS;
+    const size_t P = qs_open_parts(b->max_vocab);
+    const size_t hist = sizeof(uint64_t) * QS_OPEN_BINS * R, sum = sizeof(OpenSum) * P * R,
+                 prec = sizeof(OpenPartRec) * P * R, list = sizeof(uint64_t) * 2 * QS_OPEN_LIST * R,
+                 ctl = sizeof(OpenCtl) * R;
+    uint8_t *p = nullptr;
+    if (hipMalloc((void **)&p, hist + prec + sum + list + ctl) != hipSuccess) {
+        (void)hipGetLastError();
+        return;
+    }
+    if (hipMemset(p, 0, hist + prec + sum + list + ctl) != hipSuccess) {
+        (void)hipGetLastError();
+        (void)hipFree(p);
+        return;
+    }
+    b->d_open = p;
+    b->open.hist = (uint64_t *)p;
+    b->open.prec = (OpenPartRec *)(p + hist);
+    b->open.sum = (OpenSum *)(p + hist + prec);
+    b->open.list = (uint64_t *)(p + hist + prec + sum);
+    b->open.ctl = (OpenCtl *)(p + hist + prec + sum + list);
 }
 
 static int upload_rows(qs_batch *b, int row0, int n_rows) {
@@ -811,6 +844,7 @@ int qs_batch_config(qs_batch *b, int row0, int n_rows, float temperature, float 
         qs_clamp_config(temperature, top_p, top_k, min_p, repeat_penalty, repeat_last_n,
                         seeds ? seeds[r] : 0ull, p.ring_cap, &p, &rng[r]);
     }
+    if (qs_open_row(b->h_prm[row0], b->max_vocab)) open_alloc(b);
     int rc = upload_rows(b, row0, n_rows);
     if (rc) return rc;
     std::vector<int32_t> zero(n_rows, 0);
@@ -956,8 +990,26 @@ static int pick_range(qs_batch *b, int row0, const float *d_logits, int64_t row_
             qs_set_error("qs_batch_pick: the streaming kernel does not support this pick");
             return QS_EINVAL;
         }
-        return qs_part_launch(d_logits, row_stride, n_rows, n_vocab, st0, b->sc, d_out, d_diag,
-                              b->part_resident, b->stream, b->mid, !any_sample);
+        // rows without a top-k: the whole-window decision over several workgroups, which never
+        // waits for a scratch slot; a spin limit of 0 asks every whole-window row to give up
+        // (failure injection), so it stands aside
+        bool open = false;
+        for (int r = row0; b->d_open && b->sc.spin_limit > 0 && n_rows <= QS_OPEN_ROWS &&
+                           r < row0 + n_rows && !open; ++r)
+            open = qs_open_row(b->h_prm[r], n_vocab);
+        if (open && b->open_dirty) {
+            HIP_TRY(hipStreamSynchronize(b->stream), "sync");
+            const size_t R = b->max_rows < QS_OPEN_ROWS ? b->max_rows : QS_OPEN_ROWS;
+            HIP_TRY(hipMemset(b->open.hist, 0, sizeof(uint64_t) * QS_OPEN_BINS * R), "open rows");
+            HIP_TRY(hipMemset(b->open.ctl, 0, sizeof(OpenCtl) * R), "open rows");
+            HIP_TRY(hipStreamSynchronize(nullptr), "open rows");
+        }
+        b->open_dirty = open;
+        const int rc = qs_part_launch(d_logits, row_stride, n_rows, n_vocab, st0, b->sc, d_out,
+                                      d_diag, b->part_resident, b->stream, b->mid, !any_sample,
+                                      open ? &b->open : nullptr);
+        if (rc == 0) b->open_dirty = false;
+        return rc;
     }
     Geometry g;
     g.logits = d_logits;

@@ -16,6 +16,44 @@
 #define QS_PART_WAVES 8
 #define QS_PART_CANDS 256
 
+// The whole-window decision of rows without a top-k over several workgroups (qs_open.h):
+// logits a workgroup takes, histogram bins, entries a row's list holds, and the rows of a
+// pick it serves (larger picks decide such rows in their own workgroup).
+#define QS_OPEN_PART 4096
+#define QS_OPEN_BINS 1024
+#define QS_OPEN_LIST 4096
+#define QS_OPEN_ROWS 64
+
+// Its scratch, per row (hist, cnt and done zero between picks: the row's last part resets
+// them): the histogram of numerators' mass, per part the first pass's sums and the second
+// pass's, the two lists, and the row's control words.
+struct OpenSum {
+    double sum, m_in, m_out;         // numerators; those surely / possibly above min-p
+    int32_t cnt, pad;                // logits in the window
+};
+struct OpenPartRec {
+    double above1, above2, kept, all;    // p above the cut's and the draw's bins, at or above
+                                         // min-p's floor, and of every id
+    int32_t n1, n2, nk, pad;
+    uint32_t min1, max1, min2, max2;     // least p bits above / largest below those bins
+};
+struct OpenCtl {
+    uint64_t cnt;                    // entries of the two lists (low and high half)
+    int32_t done;                    // parts finished
+    int32_t reason;                  // 0: decided before; else the CF_* reason it is here
+    float maxl, scale;
+};
+struct OpenScratch {
+    uint64_t *hist;                  // [rows][QS_OPEN_BINS]  (null: no such scratch)
+    OpenSum *sum;                    // [rows][parts]
+    OpenPartRec *prec;               // [rows][parts]
+    uint64_t *list;                  // [rows][2][QS_OPEN_LIST]
+    OpenCtl *ctl;                    // [rows]
+};
+// Open parts a row of n_vocab logits has; whether a row's settings take this path.
+inline int qs_open_parts(int n_vocab) { return (n_vocab + QS_OPEN_PART - 1) / QS_OPEN_PART; }
+bool qs_open_row(const qs_row_param &p, int n_vocab);
+
 // Whether the streaming kernel handles this pick (16-byte aligned rows, vocabulary and row
 // stride multiples of 4, at most QS_PART_MAX_PARTS parts).
 int qs_part_supported(int n_rows, int n_vocab, int64_t row_stride, const void *logits);
@@ -28,11 +66,14 @@ int qs_part_resident(void);
 // for another).
 // `mid`, when given, is recorded on the stream between the two kernels (timing).  When
 // every row is greedy (`all_greedy`) and sc.gbest is set, each row is decided by its last
-// part in the streaming kernel and the decision kernel is not launched.
+// part in the streaming kernel and the decision kernel is not launched.  With `open` (some
+// row passes qs_open_row; the scratch for n_rows rows), rows the certified decision leaves
+// undecided take the whole-window decision over several workgroups.
 int qs_part_launch(const float *logits, int64_t row_stride, int n_rows, int n_vocab,
                    const qs::RowState &st, const qs::Scratch &sc, int32_t *out,
                    qs_pick_diag *diag, int resident, hipStream_t stream,
-                   hipEvent_t mid = nullptr, bool all_greedy = false);
+                   hipEvent_t mid = nullptr, bool all_greedy = false,
+                   const OpenScratch *open = nullptr);
 
 // ---- the row kernel (qs_row.hip) ----
 

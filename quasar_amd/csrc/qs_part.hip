@@ -37,6 +37,7 @@
 #include "qs_decide.h"
 #include "qs_device.h"
 #include "qs_launch.h"
+#include "qs_open.h"
 
 using namespace qs;
 using namespace qs::dec;
@@ -913,8 +914,25 @@ __device__ __forceinline__ int decide_par(const PartArgs &a, int row, const qs_r
                          hist);
 }
 
-__global__ void __launch_bounds__(ND) k_decide(PartArgs a) {
-    __shared__ DecLds dl;
+// The LDS of a workgroup that may take either a row's decision or a part of an open row.
+constexpr size_t OPEN_LDS =
+    sizeof(open::OpenLds) > sizeof(DecLds) ? sizeof(open::OpenLds) : sizeof(DecLds);
+
+// The row decisions.  OPEN: some row has no top-k and the scratch of qs_open.h is there;
+// rows it serves that the certified decision leaves undecided are left to k_open, and the
+// workgroups past the row decisions take those rows' first pass meanwhile (the chip is
+// otherwise idle: a decision is one workgroup a row).
+template <bool OPEN>
+__global__ void __launch_bounds__(ND) k_decide(PartArgs a, open::OpenArgs o) {
+    __shared__ __align__(16) unsigned char lds[OPEN ? OPEN_LDS : sizeof(DecLds)];
+    DecLds &dl = *(DecLds *)lds;
+    if constexpr (OPEN) {
+        if ((int)blockIdx.x >= a.n_rows) {
+            const int i = (int)blockIdx.x - a.n_rows, part = i / a.n_rows;
+            open::open_sum(a, o, i - part * a.n_rows, part, *(open::OpenLds *)lds, c_tab_part);
+            return;
+        }
+    }
     QS_DEC_MARK(0);
     const int row = blockIdx.x, tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
     const Scratch &sc = a.sc;
@@ -928,6 +946,17 @@ __global__ void __launch_bounds__(ND) k_decide(PartArgs a) {
     if (tid < QS_EXPF_TAB_N) dl.dl.tab[tid] = c_tab_part[tid];
     RowHist hist{0ull, 0, 0};
     if (tid < 64 && !greedy) hist = row_hist(st, row);
+    // a row the certified decision does not cover: left to k_open, or decided here
+    if (OPEN && tid == 0) o.s.ctl[row].reason = 0;
+    auto undecided = [&](const CertTotals &t, int reason) __attribute__((always_inline)) {
+        if constexpr (OPEN) {
+            if (open::open_row(P, a.vocab) && isfinite(t.msc)) {
+                if (tid == 0) o.s.ctl[row].reason = reason;
+                return;
+            }
+        }
+        exact_row(a, row, P, t, dl, hist, reason);
+    };
     if (NL <= 128) {
         // rows of up to 16 parts: greedy rows by wavefront 0 alone, sampling rows by the
         // workgroup (decide_par); the whole workgroup then takes the block decision, a
@@ -962,7 +991,7 @@ __global__ void __launch_bounds__(ND) k_decide(PartArgs a) {
                                         a.diag, hist);
             if (status == 0) return;
         }
-        exact_row(a, row, P, t, dl, hist, status);
+        undecided(t, status);
         return;
     }
     // records and lists tid and ND + tid (number L: wavefront L mod 8 of part L / 8, its
@@ -1140,10 +1169,19 @@ __global__ void __launch_bounds__(ND) k_decide(PartArgs a) {
         }
     }
     if (status == 0) return;
-    exact_row(a, row, P, t, dl, hist, status);
+    undecided(t, status);
+}
+
+// The second pass and the decision of the rows k_decide<true> left (qs_open.h).
+__global__ void __launch_bounds__(ND) k_open(PartArgs a, open::OpenArgs o) {
+    __shared__ __align__(16) unsigned char lds[OPEN_LDS];
+    const int part = (int)blockIdx.x / a.n_rows, row = (int)blockIdx.x - part * a.n_rows;
+    open::open_select(a, o, row, part, *(open::OpenLds *)lds, *(DecLds *)lds, c_tab_part);
 }
 
 }  // namespace
+
+bool qs_open_row(const qs_row_param &p, int n_vocab) { return open::open_row(p, n_vocab); }
 
 int qs_part_parts(int n_vocab) { return (n_vocab + PART_MAX - 1) / PART_MAX; }
 
@@ -1166,7 +1204,8 @@ int qs_part_resident(void) {
 
 int qs_part_launch(const float *logits, int64_t row_stride, int n_rows, int n_vocab,
                    const RowState &st, const Scratch &sc, int32_t *out, qs_pick_diag *diag,
-                   int resident, hipStream_t stream, hipEvent_t mid, bool all_greedy) {
+                   int resident, hipStream_t stream, hipEvent_t mid, bool all_greedy,
+                   const OpenScratch *open) {
     PartArgs a;
     a.logits = logits;
     a.stride = row_stride;
@@ -1220,8 +1259,23 @@ int qs_part_launch(const float *logits, int64_t row_stride, int n_rows, int n_vo
     hipError_t e = hipGetLastError();
     if (e == hipSuccess && mid) e = hipEventRecord(mid, stream);
     if (e == hipSuccess && !gf) {
-        hipLaunchKernelGGL(k_decide, dim3((unsigned)n_rows), dim3(ND), 0, stream, a);
-        e = hipGetLastError();
+        open::OpenArgs oa{};
+        if (open) {
+            oa.s = *open;
+            oa.parts = qs_open_parts(n_vocab);
+            const unsigned np = (unsigned)(n_rows * oa.parts);
+            hipLaunchKernelGGL(k_decide<true>, dim3((unsigned)n_rows + np), dim3(ND), 0, stream,
+                               a, oa);
+            e = hipGetLastError();
+            if (e == hipSuccess) {
+                hipLaunchKernelGGL(k_open, dim3(np), dim3(ND), 0, stream, a, oa);
+                e = hipGetLastError();
+            }
+        } else {
+            hipLaunchKernelGGL(k_decide<false>, dim3((unsigned)n_rows), dim3(ND), 0, stream, a,
+                               oa);
+            e = hipGetLastError();
+        }
     }
     if (e != hipSuccess) {
         qs_set_error("streaming pick launch: %s", hipGetErrorString(e));

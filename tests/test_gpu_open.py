@@ -1,0 +1,76 @@
+"""GPU: rows without a top-k whose kept prefix may be the whole window (qs_open.h), against
+the CPU restatement (sample.c:111-179) on the same logits: ids, the kept prefixes, the
+drawn position, the softmax normaliser, generator states and histories.  All whole numbers
+(inv: a float fixed by the definition), so compared exactly."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+# vocabularies at the part's edges (4,096 logits) and over the real range
+SIZES = [4, 60, 4092, 4096, 4100, 40960, 151936, 262144]
+# (temperature, top_p, top_k, min_p, penalty, last_n)
+SETTINGS = [
+    (1.0, 1.0, 0, 0.0, 1.0, 0), (0.7, 0.9, 0, 0.0, 1.0, 0), (1.0, 0.8, 0, 0.1, 1.2, 64),
+    (1.0, 1.0, 0, 0.1, 1.0, 0), (1.3, 0.9999999, 0, 0.0, 1.0, 0), (1.0, 0.95, 1 << 30, 0.0, 1.3, 16),
+    (0.05, 1.0, 0, 1e-6, 1.0, 0), (1.0, 1.0, 0, 2.0, 1.0, 0),
+]
+
+
+def rows_of(V, seed):
+    """Flat, wide, narrow, peaked and heavy-tailed rows, rows on a bf16 grid, one value only,
+    and rows with infinities and NaN."""
+    r = np.random.default_rng(seed)
+    x = r.normal(0, 2, (10, V)).astype(np.float32)
+    x[1] = r.normal(0, 1, V)
+    x[2] = r.normal(0, 0.01, V)
+    x[3, r.integers(V)] += 12
+    x[4] = r.standard_t(3, V) * 2
+    bf = (r.normal(0, 2, V).astype(np.float32).view(np.uint32) + 0x8000) & 0xFFFF0000
+    x[5] = bf.astype(np.uint32).view(np.float32)
+    x[6] = 0.25
+    x[7, ::3] = -np.inf
+    x[8, V // 2] = np.nan
+    x[9] = np.round(x[9])
+    return x
+
+
+@pytest.mark.parametrize("V", SIZES)
+def test_open_rows(oracle, V):
+    import quasar_amd as qa
+    x = rows_of(V, V)
+    B = len(SETTINGS) * len(x)
+    n = min(B, 64)
+    full = np.concatenate([x] * len(SETTINGS))
+    for first in range(0, B, n):
+        m = min(n, B - first)
+        b = qa.Batch(n, V, 64)
+        buf = qa.DeviceBuffer.from_array(full[first:first + m])
+        b.set_mode(2)
+        hist = np.random.default_rng(V + first).integers(0, V, (m, 24)).astype(np.int32)
+        for r in range(m):
+            b.config(r, 1, *SETTINGS[(first + r) // len(x)], seeds=[1000 + first + r])
+        b.set_history(0, hist)
+        got = [b.pick(buf.ptr, V, m, V, diag=True) for _ in range(2)]
+        paths = {}
+        for r in range(m):
+            s = oracle.sampler()
+            cfg = SETTINGS[(first + r) // len(x)]
+            s.config(*cfg, seed=1000 + first + r)
+            s.set_history(hist[r])
+            for k in range(2):
+                want, od = s.pick_diag(full[first + r])
+                ids, d = got[k][0], got[k][1][r]
+                at = (V, cfg, r % len(x), k, d.path, d.fallback)
+                assert int(ids[r]) == want, at
+                assert d.keep == od["keep"], at
+                if d.path == qa.PATH_FULL:
+                    assert np.float32(d.inv) == np.float32(od["inv"]) or np.isnan(od["inv"]), at
+                    assert (d.keep_topp, d.n_window, d.rank) == \
+                        (od["keep_topp"], od["n_window"], od["rank"]), at
+                paths[d.path] = paths.get(d.path, 0) + 1
+            rng, h = b.get_state(r)
+            assert rng == s.rng and (h == s.history()).all(), at
+        print(V, first, "paths", paths, flush=True)
+        b.close()
+        buf.free()
