@@ -164,9 +164,9 @@ int qs_batch_pick_rows(qs_batch *b, int row0, const float *d_logits, int64_t row
                        int n_rows, int n_vocab, int32_t *d_out, qs_pick_diag *d_diag);
 
 /* Which kernels qs_batch_pick uses.  AUTO (the default) takes the row kernel for batches
- * of at least one row per CU whose sampling rows have a top-k of at most 256 (or top-k
- * off), the streaming kernels for smaller batches and larger top-k, and the split-row
- * kernels for rows neither supports.  ROW: one kernel, one workgroup per row,
+ * of at least a quarter of a row per CU whose sampling rows have a top-k of at most 256 (or top-k
+ * off), the streaming kernels for smaller batches, larger top-k and rows at any other
+ * alignment, and the split-row kernels for vocabularies neither supports.  ROW: one kernel, one workgroup per row,
  * every logit read once and the row decided from LDS (16-byte aligned rows, a vocabulary
  * and a row stride that are multiples of 4, vocabulary up to 262,144).  STREAM: two
  * kernels, every logit read once by workgroups that each take a part of a row, then one

@@ -669,7 +669,7 @@ static int batch_alloc(qs_batch *b) {
     int sr = R;
     const int many = TARGET_WGS < S_MAX * R ? TARGET_WGS : S_MAX * R;
     if (many > sr) sr = many;
-    const int np = qs_part_parts(V);
+    const int np = qs_part_parts(V + 3);     // (rows at any alignment: their shift)
     if ((int64_t)np * R > sr) sr = np * R;
     b->slice_rows = sr;
     b->part_resident = qs_part_resident();
@@ -770,7 +770,9 @@ static bool rows_ok(const qs_batch *b, int row0, int n_rows) {
 // kernel when the batch has a row for at least a quarter of the CUs and every sampling row
 // aims at most QS_ROW_AUTO_KSEL candidates (its per-wavefront candidate lists hold a few
 // hundred entries; a row that overflows them takes the full-window path), the streaming
-// kernels when the rows allow them, the split-row kernels otherwise.  `kmax` is the largest
+// kernels otherwise (rows at any alignment; the split-row kernels took 44 us for 48 rows of
+// 100,003 logits where they take 21), the split-row kernels for vocabularies below 4 or past
+// their parts.  `kmax` is the largest
 // candidate target among the sampling rows (1 when every row is greedy).  The quarter: on
 // MI355X (256 CUs) at 151,936 logits a row, a pick of the row kernel takes about 23 us
 // from 8 to 64 rows (one workgroup per row, each row's latency), the streaming pair 17 us at
@@ -781,8 +783,10 @@ static int auto_mode(const qs_batch *b, const float *d_logits, int64_t row_strid
     if (4 * (int64_t)n_rows >= b->n_cu && kmax <= QS_ROW_AUTO_KSEL &&
         qs_row_supported(n_rows, n_vocab, row_stride, d_logits))
         return QS_MODE_ROW;
-    return qs_part_supported(n_rows, n_vocab, row_stride, d_logits) ? QS_MODE_STREAM
-                                                                    : QS_MODE_SPLIT;
+    return qs_part_supported(n_rows, n_vocab, row_stride, d_logits) ||
+                   qs_part_takes(n_rows, n_vocab, d_logits)
+               ? QS_MODE_STREAM
+               : QS_MODE_SPLIT;
 }
 
 // Wavefronts per row of the row kernel: 16 (one workgroup per CU) up to a row per CU, 8
@@ -986,7 +990,8 @@ static int pick_range(qs_batch *b, int row0, const float *d_logits, int64_t row_
                              row_waves(b, n_rows), b->stream);
     }
     if (mode == QS_MODE_STREAM) {
-        if (!qs_part_supported(n_rows, n_vocab, row_stride, d_logits)) {
+        if (b->mode == QS_MODE_STREAM &&
+            !qs_part_supported(n_rows, n_vocab, row_stride, d_logits)) {
             qs_set_error("qs_batch_pick: the streaming kernel does not support this pick");
             return QS_EINVAL;
         }

@@ -83,10 +83,26 @@ struct DecLds {
 };
 static_assert(sizeof(FullLds<ND>) <= sizeof(uint32_t) * 2 * FCAP, "full-window LDS aliases keys/ids");
 
+// Floats before a row's first logit in its 16-byte group.  Rows at any alignment are read
+// in whole groups from that group on (a group holding a byte of the row lies in a page of
+// it), at positions v = id + shift; the positions before the row and past it are masked.
+__host__ __device__ __forceinline__ int row_shift(const float *logits, int64_t stride, int row) {
+    return (int)(((uintptr_t)(logits + (int64_t)row * stride) >> 2) & 3u);
+}
+
+// Logits of the row in part j (parts are part_len positions).
+template <bool UNAL>
+__device__ __forceinline__ int part_count(const PartArgs &a, int row, int j) {
+    if (!UNAL) return min(a.part_len, a.vocab - j * a.part_len);
+    const int sh = row_shift(a.logits, a.stride, row);
+    const int lo = max(j * a.part_len, sh), hi = min((j + 1) * a.part_len, a.vocab + sh);
+    return max(hi - lo, 0);
+}
+
 // Visit the row's penalised logits (f(w, id) on every thread's share; all threads): in
 // blocks of XBM logits, each with its history bitmap in LDS, read XUP float4s per thread at
-// a time with every load issued before the first is used.
-template <typename F>
+// a time with every load issued before the first is used.  UNAL: rows at any alignment.
+template <bool UNAL, typename F>
 __device__ __forceinline__ void row_visit(const PartArgs &a, int row, const qs_row_param &P,
                                           DecLds &dl, F &&f) {
     const int tid = threadIdx.x;
@@ -96,15 +112,17 @@ __device__ __forceinline__ void row_visit(const PartArgs &a, int row, const qs_r
     ring_pos(a.st, row, cap, len, head);
     const bool pen = rp > 1.0f && len > 0 && cap > 0;
     const int32_t *ring = a.st.ring + (int64_t)row * a.st.ring_stride;
-    const float4 *x4 = (const float4 *)(a.logits + (int64_t)row * a.stride);
-    for (int lo = 0; lo < a.vocab; lo += XBM) {
-        const int hi = min(lo + XBM, a.vocab), c_hi = hi >> 2;
+    const int sh = UNAL ? row_shift(a.logits, a.stride, row) : 0, end = a.vocab + sh;
+    const float4 *x4 = (const float4 *)(a.logits + (int64_t)row * a.stride - sh);
+    for (int lo = 0; lo < end; lo += XBM) {
+        const int hi = min(lo + XBM, end), c_hi = UNAL ? (hi + 3) >> 2 : hi >> 2;
         if (pen) {                                    // sample.c:118-120: each id once
             for (int j = tid; j < bitmap_words(XBM); j += ND) dl.bm[j] = 0u;
             __syncthreads();
             for (int j = tid; j < len; j += ND) {
                 const int id = ring[qs_ring_slot(cap, head, j)];
-                if (id >= lo && id < hi) atomicOr(&dl.bm[(id - lo) >> 5], 1u << ((id - lo) & 31));
+                const int q = id - (lo - sh);
+                if (id >= lo - sh && id < hi - sh) atomicOr(&dl.bm[q >> 5], 1u << (q & 31));
             }
             __syncthreads();
         }
@@ -124,8 +142,9 @@ __device__ __forceinline__ void row_visit(const PartArgs &a, int row, const qs_r
                 const uint32_t nib = pen ? (dl.bm[q >> 5] >> (q & 31)) & 0xFu : 0u;
 #pragma unroll
                 for (int e = 0; e < 4; ++e) {
+                    if (UNAL && (4 * c + e < sh || 4 * c + e >= end)) continue;
                     if ((nib >> e) & 1u) w[e] = penalise(w[e], rp);
-                    f(w[e], 4 * c + e);
+                    f(w[e], 4 * c + e - sh);
                 }
             }
         }
@@ -141,13 +160,14 @@ __device__ __forceinline__ void row_visit(const PartArgs &a, int row, const qs_r
 // (float)(1 / x) is the same float at both ends of that reach it is the reference's inv
 // (1 / x and both roundings are monotone), and where it is not (or sc.sum_in_order asks
 // for it) the sum is taken again in id order.
+template <bool UNAL = false>
 __device__ __forceinline__ void exact_totals(const PartArgs &a, int row, const qs_row_param &P, float msc,
                              DecLds &dl, double &sum, int &nwin) {
     const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
     const float inv_t = P.inv_t, thr = msc - 30.0f;
     double acc = 0.0;
     int cnt = 0;
-    row_visit(a, row, P, dl, [&](float w, int) {
+    row_visit<UNAL>(a, row, P, dl, [&](float w, int) {
         const float s = w * inv_t;
         if (s >= thr) {
             acc += (double)qs_expf_core(s - msc, dl.dl.tab);
@@ -184,6 +204,7 @@ __device__ __forceinline__ void block_best(float &v, int &i, DecLds &dl) {
 // The exact path (all threads): the row's exact denominator, then the reference's decision
 // over the gathered candidates (or the whole window); `status` is the reason the certified
 // decision gave up, kept in the diagnostics.
+template <bool UNAL = false>
 __device__ __forceinline__ void exact_row(const PartArgs &a, int row, const qs_row_param &P,
                                           const CertTotals &t, DecLds &dl, const RowHist &hist,
                                           int status) {
@@ -195,7 +216,7 @@ __device__ __forceinline__ void exact_row(const PartArgs &a, int row, const qs_r
     rt.cflag = t.cflag;
     rt.rej = t.rej;
     rt.total = t.total;
-    if (isfinite(t.msc)) exact_totals(a, row, P, t.msc, dl, rt.sum, rt.nwin);
+    if (isfinite(t.msc)) exact_totals<UNAL>(a, row, P, t.msc, dl, rt.sum, rt.nwin);
     QS_DEC_MARK(5);
     decide_row_fast<ND, SCAP, false>(row, P, rt, FCAP, dl.keys, dl.ids, dl.srt, dl.dl, fl,
                                      a.logits + (int64_t)row * a.stride, a.vocab, a.st, a.sc,

@@ -453,6 +453,7 @@ __device__ __forceinline__ bool open_finish(const PartArgs &a, const OpenArgs &o
 }
 
 // The second pass: one part of a row whose decision kernel left it here.
+template <bool UNAL>
 __device__ __forceinline__ void open_select(const PartArgs &a, const OpenArgs &o, int row,
                                             int part, OpenLds &L, DecLds &dl,
                                             const uint64_t *ctab) {
@@ -676,7 +677,7 @@ __device__ __forceinline__ void open_select(const PartArgs &a, const OpenArgs &o
     __syncthreads();
     double sum = 0.0;
     int nw = 0;
-    dec::exact_totals(a, row, P, msc, dl, sum, nw);
+    dec::exact_totals<UNAL>(a, row, P, msc, dl, sum, nw);
     full_row<ND>(a.logits + (int64_t)row * a.stride, a.vocab, row, P, maxl, sum, a.st, a.sc,
                  a.out, a.diag, dl.dl.tab, *(FullLds<ND> *)dl.keys, -1);
     __syncthreads();

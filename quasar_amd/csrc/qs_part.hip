@@ -1,7 +1,10 @@
 // qs_part.hip - the streaming pick: one workgroup per part of a row, every logit read once,
 // then one workgroup per row for the decision.
 //
-// A pick of B rows of V logits (sample.c:111-179 per row) is two kernels:
+// A pick of B rows of V logits (sample.c:111-179 per row) is two kernels (rows that are not
+// 16-byte aligned are read in whole 16-byte groups with the positions outside the row masked:
+// 48 rows of 100,003 logits, ids on the host, 90 us a pick through the split kernels' two
+// scalar passes, 59 us here):
 //
 // k_part, B x P workgroups of 512 threads, P = ceil(V / 10240) parts per row (15 at
 // V = 151,936).  A workgroup holds its part in registers (five float4 per thread, the
@@ -115,18 +118,27 @@ struct PartLds {
     uint64_t gbw[2][NWV];            // greedy rows: per-wave (key, ~id) best, by parity
 };
 
-struct Loc {                          // a part of a row
-    int row, part, lo, hi, c_lo, c_hi;
+// A part of a row, in positions v = id + sh (row_shift; sh is 0 for 16-byte aligned rows) and
+// in float4s of them.  UNAL (rows at any alignment): the positions below sh, in the row's
+// first float4, and from vocab + sh on, in its last, are not logits.
+struct Loc {
+    int row, part, lo, hi, c_lo, c_hi, sh;
 };
-__device__ __forceinline__ Loc part_loc(int part_len, int vocab, int row, int part) {
+template <bool UNAL>
+__device__ __forceinline__ Loc part_loc(const StreamArgs &a, int row, int part) {
     Loc l;
     l.row = row;
     l.part = part;
-    l.lo = part * part_len;
-    l.hi = min(l.lo + part_len, vocab);
+    l.sh = UNAL ? row_shift(a.logits, a.stride, row) : 0;
+    l.lo = part * a.part_len;
+    l.hi = min(l.lo + a.part_len, a.vocab + l.sh);
+    if (UNAL) l.hi = max(l.hi, l.lo);        // a last part that this row's shift leaves empty
     l.c_lo = l.lo >> 2;
-    l.c_hi = l.hi >> 2;
+    l.c_hi = UNAL ? (l.hi + 3) >> 2 : l.hi >> 2;
     return l;
+}
+__device__ __forceinline__ bool is_logit(const StreamArgs &a, const Loc &l, int v) {
+    return v >= l.sh && v < a.vocab + l.sh;
 }
 
 // The parts of the pick are dealt to the grid's workgroups in contiguous runs.  With
@@ -155,14 +167,16 @@ __device__ __forceinline__ Run my_run(const StreamArgs &a) {
     }
     return r;
 }
+template <bool UNAL>
 __device__ __forceinline__ Loc part_at(const StreamArgs &a, const Run &r, int idx) {
     const int q = idx / a.parts, j = idx - q * a.parts;
-    return part_loc(a.part_len, a.vocab, r.xcd >= 0 ? q * 8 + r.xcd : q, j);
+    return part_loc<UNAL>(a, r.xcd >= 0 ? q * 8 + r.xcd : q, j);
 }
 // The part after l in a run (no division).
+template <bool UNAL>
 __device__ __forceinline__ Loc loc_next(const StreamArgs &a, const Run &r, const Loc &l) {
-    return l.part + 1 < a.parts ? part_loc(a.part_len, a.vocab, l.row, l.part + 1)
-                                : part_loc(a.part_len, a.vocab, l.row + (r.xcd >= 0 ? 8 : 1), 0);
+    return l.part + 1 < a.parts ? part_loc<UNAL>(a, l.row, l.part + 1)
+                                : part_loc<UNAL>(a, l.row + (r.xcd >= 0 ? 8 : 1), 0);
 }
 
 // The part's logits into the LDS staging buffer: a buffer resource over its float4s; float4
@@ -173,7 +187,7 @@ constexpr int BUF_WORD3 = 0x00020000;    // raw buffer, 32-bit data format
 constexpr int BUF_NT = 2;                // nontemporal: each logit is read once
 typedef __attribute__((address_space(3))) void lds_void;
 __device__ __forceinline__ void issue_stage(float4 *stage, const StreamArgs &a, const Loc &l) {
-    const float *base = a.logits + (int64_t)l.row * a.stride + 4 * (int64_t)l.c_lo;
+    const float *base = a.logits + (int64_t)l.row * a.stride - l.sh + 4 * (int64_t)l.c_lo;
     const __amdgpu_buffer_rsrc_t rs =
         __builtin_amdgcn_make_buffer_rsrc((void *)base, 0, (l.c_hi - l.c_lo) * 16, BUF_WORD3);
     const int tid = tix();
@@ -222,8 +236,9 @@ __device__ __forceinline__ void bitmap_mark(uint32_t *bm, uint32_t *hitw, const 
     int len = a.hlen[l.row], head = a.hhead[l.row];
     qs_ring_clamp(cap, &len, &head);
     auto mark = [&](int p, int id) {
-        if (qs_ring_live(cap, len, head, p) && id >= l.lo && id < l.hi) {
-            const int q = id - l.lo, c = q >> 2, u = c / NT;   // float4 c: thread c - u*NT
+        if (qs_ring_live(cap, len, head, p) && id >= l.lo - l.sh && id < l.hi - l.sh) {
+            const int q = id - (l.lo - l.sh), c = q >> 2, u = c / NT;   // float4 c: thread
+                                                                        // c - u*NT
             lds_or(&bm[q >> 5], 1u << (q & 31));
             lds_or(&hitw[(c - u * NT) >> 6], 1u << u);
         }
@@ -264,6 +279,11 @@ __device__ __forceinline__ void bitmap_zero(uint32_t *bm, uint32_t *hitw) {
 __device__ __forceinline__ bool wave_tail(const Loc &l, int u, int wv) {
     return l.c_lo + u * NT + wv * 64 + 63 >= l.c_hi;
 }
+// UNAL: whether it holds positions that are not logits (a uniform test).
+__device__ __forceinline__ bool wave_edge(const StreamArgs &a, const Loc &l, int u, int wv) {
+    const int c = l.c_lo + u * NT + wv * 64;
+    return c == 0 || c + 63 >= (a.vocab + l.sh) >> 2;
+}
 
 // Pass 1: penalty, each thread's max and min over non-NaN logits, its NaN count.  Positions
 // past the part become -inf in the registers; NaNs stay (no >= test passes them and the
@@ -272,9 +292,10 @@ struct Pass1 {
     float mx, mn;                    // max / min over the thread's logits (min: non-NaN)
     int nan;                         // NaNs among them
 };
-template <bool TAIL>
-__device__ __forceinline__ Pass1 pass1(float4 (&buf)[UP], const Loc &l, const uint32_t *bm,
-                                       const uint32_t *hitw, bool pen, float rp, int wv) {
+template <bool TAIL, bool UNAL>
+__device__ __forceinline__ Pass1 pass1(float4 (&buf)[UP], const StreamArgs &a, const Loc &l,
+                                       const uint32_t *bm, const uint32_t *hitw, bool pen,
+                                       float rp, int wv) {
     const int tid = tix();
     const uint32_t *bw = bm + (tid >> 3);             // word (u*NT + tid)/8, NT % 8 == 0
     const uint32_t bsh = (uint32_t)(tid & 7) * 4u;
@@ -291,7 +312,14 @@ __device__ __forceinline__ Pass1 pass1(float4 (&buf)[UP], const Loc &l, const ui
                     if ((nib >> k) & 1u) w[k] = penalise(w[k], rp);
             }
         }
-        if (TAIL && wave_tail(l, u, wv)) {           // a scalar branch: tail waves only
+        if (UNAL && wave_edge(a, l, u, wv)) {
+#pragma unroll
+            for (int k = 0; k < 4; ++k) {
+                const bool in = is_logit(a, l, 4 * (l.c_lo + u * NT + tid) + k);
+                if (!in) w[k] = -INFINITY;
+                else r.mn = __builtin_elementwise_minimum(r.mn, w[k]);
+            }
+        } else if (!UNAL && TAIL && wave_tail(l, u, wv)) {           // a scalar branch: tail waves only
             if (l.c_lo + u * NT + tid >= l.c_hi) w[0] = w[1] = w[2] = w[3] = -INFINITY;
             else r.mn = min3n(min3n(r.mn, w[0], w[1]), w[2], w[3]);
         } else {
@@ -311,7 +339,8 @@ __device__ __forceinline__ Pass1 pass1(float4 (&buf)[UP], const Loc &l, const ui
             for (int k = 0; k < 4; ++k) {
                 r.nan += w[k] != w[k];
                 r.mx = w[k] > r.mx ? w[k] : r.mx;
-                r.mn = (w[k] < r.mn && !tail) ? w[k] : r.mn;
+                const bool out = UNAL ? !is_logit(a, l, 4 * (l.c_lo + u * NT + tid) + k) : tail;
+                r.mn = (w[k] < r.mn && !out) ? w[k] : r.mn;
             }
         }
     }
@@ -356,7 +385,7 @@ __device__ __forceinline__ int part_m(const qs_row_param &P, int parts) {
 // barrier, then `mid` (the caller's bitmap upkeep), the part's max and threshold, the sums
 // (sampling rows), the candidates and the wavefront's record.  Nothing here waits for
 // another wavefront after the barrier.
-template <bool GF, typename Mid>
+template <bool GF, bool UNAL, typename Mid>
 __device__ __forceinline__ void part_step(float4 (&buf)[UP], const StreamArgs &a, const Loc &l,
                                           const qs_row_param &P, const uint32_t *bm,
                                           const uint32_t *hitw, int par, PartLds &pl, Mid &&mid,
@@ -370,11 +399,13 @@ __device__ __forceinline__ void part_step(float4 (&buf)[UP], const StreamArgs &a
     // of the wavefronts with such positions floor t
     TL_PART(tl, 1);
     const bool tailp = l.c_hi - l.c_lo < NT * UP;
-    const Pass1 r = tailp ? pass1<true>(buf, l, bm, hitw, pen, rp, wv)
-                          : pass1<false>(buf, l, bm, hitw, pen, rp, wv);
+    const Pass1 r = tailp ? pass1<true, UNAL>(buf, a, l, bm, hitw, pen, rp, wv)
+                          : pass1<false, UNAL>(buf, a, l, bm, hitw, pen, rp, wv);
     const float inv_t = P.inv_t;
     const bool greedy = row_greedy(P);
-    const bool dirty = (tailp && wave_tail(l, UP - 1, wv)) ||
+    // (UNAL: a row's first and last parts hold positions that are not logits)
+    const bool ends = UNAL && (l.part == 0 || l.c_lo + NT * UP > (a.vocab + l.sh) >> 2);
+    const bool dirty = ends || (tailp && wave_tail(l, UP - 1, wv)) ||
                        __ballot(!(r.mn * inv_t >= SC_SANE) || r.nan != 0) != 0ull;
     const uint32_t tmk = f2key(r.mx);
     const uint32_t wmx = wave_max_u(tmk);
@@ -403,8 +434,10 @@ __device__ __forceinline__ void part_step(float4 (&buf)[UP], const StreamArgs &a
 #pragma unroll
             for (int k = 0; k < 4; ++k) {
                 const uint32_t wk = f2key(w[k] == 0.0f ? 0.0f : w[k]);
-                const uint64_t gk = ((uint64_t)wk << 32) | (uint32_t)~(uint32_t)(4 * c + k);
-                if (c < l.c_hi && w[k] == w[k] && gk > g) g = gk;
+                const uint64_t gk =
+                    ((uint64_t)wk << 32) | (uint32_t)~(uint32_t)(4 * c + k - l.sh);
+                const bool in = UNAL ? is_logit(a, l, 4 * c + k) : c < l.c_hi;
+                if (in && w[k] == w[k] && gk > g) g = gk;
             }
         }
         g = wave_reduce(g, [](uint64_t x, uint64_t y) { return x > y ? x : y; });
@@ -472,7 +505,7 @@ __device__ __forceinline__ void part_step(float4 (&buf)[UP], const StreamArgs &a
                 const uint64_t m = __ballot(hit);
                 if (m == 0ull) continue;
                 const int pos = wn + lane_prefix(m);
-                if (hit && pos < WCAP) lc[pos] = make_uint2(f2key(w[k]), (uint32_t)(4 * c + k));
+                if (hit && pos < WCAP) lc[pos] = make_uint2(f2key(w[k]), (uint32_t)(4 * c + k - l.sh));
                 wn += __popcll(m);
             }
         }
@@ -514,7 +547,7 @@ __device__ __forceinline__ void flush_part(const StreamArgs &a, PartLds &pl, int
 // lengths and heads (uniform addresses) are scalar loads, which the wavefront waits for
 // without waiting for the logit loads in flight.  They are written only by a greedy row's
 // last part (GF), through other pointers, once every part of the row has read them.
-template <bool GF>
+template <bool GF, bool UNAL>
 __global__ void __launch_bounds__(NT, 6)
 k_part(StreamArgs sa, const float *__restrict__ logits, const qs_row_param *__restrict__ prm,
        const int32_t *__restrict__ ring, const int32_t *__restrict__ hlen,
@@ -535,14 +568,14 @@ k_part(StreamArgs sa, const float *__restrict__ logits, const qs_row_param *__re
     // Every staging load batch of a part after the first goes out right behind that part's
     // ring slot load: six vector memory operations, so a wavefront waiting for the batch
     // before them waits with vmcnt(6) while they stay in flight.
-    Loc cur = part_at(a, run, run.begin);
+    Loc cur = part_at<UNAL>(a, run, run.begin);
     const int ring0 = ring_slot(a, cur.row);
     issue_stage(stage0, a, cur);
     for (int s = 0; s < 3; ++s) bitmap_zero(pl.bm[s], pl.hitw[s]);
     lds_barrier();
     bitmap_mark(pl.bm[0], pl.hitw[0], a, cur, ring0, mark_cap(a, cur.row));
     if (run.begin + 1 < run.end) {
-        const Loc n1 = loc_next(a, run, cur);
+        const Loc n1 = loc_next<UNAL>(a, run, cur);
         const int ring1 = ring_slot(a, n1.row);
         if constexpr (STAGES > 1) issue_stage(stage1, a, n1);
         bitmap_mark(pl.bm[1], pl.hitw[1], a, n1, ring1, mark_cap(a, n1.row));
@@ -570,9 +603,9 @@ k_part(StreamArgs sa, const float *__restrict__ logits, const qs_row_param *__re
         int ring_val;                                 // set (and only read) with more2; no
         if (more) {                                   // initial value, which would have to
                                                       // wait for last part's ring load
-            n1 = loc_next(a, run, cur);
+            n1 = loc_next<UNAL>(a, run, cur);
             if (more2) {
-                n2 = loc_next(a, run, n1);
+                n2 = loc_next<UNAL>(a, run, n1);
                 ring_val = ring_slot(a, n2.row);
                 if constexpr (STAGES > 1) issue_stage(stage, a, n2);
             }
@@ -580,7 +613,7 @@ k_part(StreamArgs sa, const float *__restrict__ logits, const qs_row_param *__re
         }
         const qs_row_param P = stream_param(a, cur.row);
         const int s2 = s0 == 0 ? 2 : s0 - 1;          // (s0 + 2) mod 3
-        part_step<GF>(X, a, cur, P, pl.bm[s0], pl.hitw[s0], (idx - run.begin) & 1, pl, [&] {
+        part_step<GF, UNAL>(X, a, cur, P, pl.bm[s0], pl.hitw[s0], (idx - run.begin) & 1, pl, [&] {
             // slot s0 was read by this part's pass 1 (done): cleared for part idx + 3;
             // slot s2 (cleared a part ago) gets part idx + 2's ids
             bitmap_zero(pl.bm[s0], pl.hitw[s0]);
@@ -606,8 +639,9 @@ k_part(StreamArgs sa, const float *__restrict__ logits, const qs_row_param *__re
 // Row totals from the parts' aggregates held by lanes 0..NP-1 (one wavefront): the row's
 // max, the certified denominator interval, the window size when every part lies wholly in or
 // out of the window, the largest rejected key.
-__device__ __forceinline__ CertTotals row_totals(const PartArgs &a, const qs_row_param &P,
-                                                 bool greedy, bool have, uint32_t mk,
+template <bool UNAL>
+__device__ __forceinline__ CertTotals row_totals(const PartArgs &a, int row,
+                                                 const qs_row_param &P, bool greedy, bool have, uint32_t mk,
                                                  double psum, float pterm, uint32_t pmn,
                                                  int pnan, uint32_t prej) {
     const int lane = threadIdx.x & 63;
@@ -619,7 +653,7 @@ __device__ __forceinline__ CertTotals row_totals(const PartArgs &a, const qs_row
     const float maxw = have ? key2f(mk > KEY_NEG_INF ? mk : KEY_NEG_INF) : -INFINITY;
     if (!greedy && have) cp = cert_part(maxw, psum, pterm, inv_t, msc, thr);
     const double lo = wave_sum_d(cp.lo), hi = wave_sum_d(cp.hi);
-    const int plen = have ? min(a.part_len, a.vocab - lane * a.part_len) : 0;
+    const int plen = have ? part_count<UNAL>(a, row, lane) : 0;
     const bool out_j = !(maxw * inv_t >= thr);
     const bool in_j = have && pmn != 0xFFFFFFFFu && key2f(pmn) * inv_t >= thr;
     const bool known = __ballot(have && !out_j && !in_j) == 0ull;
@@ -661,6 +695,7 @@ enum { DS_DONE = 0, DS_BLOCK = 100, DS_SCAN = 101 };
 // Returns DS_DONE, DS_BLOCK (the block decision or the exact path must run: dl.ct and the
 // gathered candidates are in place), DS_SCAN (a greedy row whose lists overflowed), or a
 // CF_* reason (dl.ct and the candidates in place).
+template <bool UNAL>
 __device__ __forceinline__ int decide_wave0(const PartArgs &a, int row, const qs_row_param &P,
                                             DecLds &dl, const RowHist &hist) {
     constexpr int SPEC = 8;
@@ -724,7 +759,7 @@ __device__ __forceinline__ int decide_wave0(const PartArgs &a, int row, const qs
     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
     __builtin_amdgcn_wave_barrier();
     const bool have = lane < NP;
-    CertTotals t = row_totals(a, P, greedy, have, have ? dl.pmaxk[lane] : 0u,
+    CertTotals t = row_totals<UNAL>(a, row, P, greedy, have, have ? dl.pmaxk[lane] : 0u,
                               have ? dl.psum[lane] : 0.0, have ? dl.pterm[lane] : 0.0f,
                               have ? dl.pmin[lane] : 0xFFFFFFFFu, have ? dl.pnan[lane] : 0,
                               have ? dl.prej[lane] : 0u);
@@ -796,6 +831,7 @@ __device__ __forceinline__ int decide_wave0(const PartArgs &a, int row, const qs
 // then wavefront 0 takes the certified decision (cert_row_wave).  All threads call it;
 // returns (in wavefront 0) DS_DONE, DS_BLOCK (the block decision or the exact path must
 // run), or a CF_* reason, with dl.ct and the gathered candidates in place.
+template <bool UNAL>
 __device__ __forceinline__ int decide_par(const PartArgs &a, int row, const qs_row_param &P,
                                           DecLds &dl, const RowHist &hist) {
     const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
@@ -860,7 +896,7 @@ __device__ __forceinline__ int decide_par(const PartArgs &a, int row, const qs_r
         asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
         __builtin_amdgcn_wave_barrier();
         const bool have = lane < NP;
-        CertTotals t = row_totals(a, P, false, have, have ? dl.pmaxk[lane] : 0u,
+        CertTotals t = row_totals<UNAL>(a, row, P, false, have, have ? dl.pmaxk[lane] : 0u,
                                   have ? dl.psum[lane] : 0.0, have ? dl.pterm[lane] : 0.0f,
                                   have ? dl.pmin[lane] : 0xFFFFFFFFu, have ? dl.pnan[lane] : 0,
                                   have ? dl.prej[lane] : 0u);
@@ -921,8 +957,8 @@ constexpr size_t OPEN_LDS =
 // The row decisions.  OPEN: some row has no top-k and the scratch of qs_open.h is there;
 // rows it serves that the certified decision leaves undecided are left to k_open, and the
 // workgroups past the row decisions take those rows' first pass meanwhile (the chip is
-// otherwise idle: a decision is one workgroup a row).
-template <bool OPEN>
+// otherwise idle: a decision is one workgroup a row).  UNAL: rows at any alignment.
+template <bool OPEN, bool UNAL>
 __global__ void __launch_bounds__(ND) k_decide(PartArgs a, open::OpenArgs o) {
     __shared__ __align__(16) unsigned char lds[OPEN ? OPEN_LDS : sizeof(DecLds)];
     DecLds &dl = *(DecLds *)lds;
@@ -955,7 +991,7 @@ __global__ void __launch_bounds__(ND) k_decide(PartArgs a, open::OpenArgs o) {
                 return;
             }
         }
-        exact_row(a, row, P, t, dl, hist, reason);
+        exact_row<UNAL>(a, row, P, t, dl, hist, reason);
     };
     if (NL <= 128) {
         // rows of up to 16 parts: greedy rows by wavefront 0 alone, sampling rows by the
@@ -963,11 +999,11 @@ __global__ void __launch_bounds__(ND) k_decide(PartArgs a, open::OpenArgs o) {
         // greedy row's scan or the exact path
         if (greedy) {
             if (wv == 0) {
-                const int s0 = decide_wave0(a, row, P, dl, hist);
+                const int s0 = decide_wave0<UNAL>(a, row, P, dl, hist);
                 if (lane == 0) dl.dl.sh[7] = s0;
             }
         } else {
-            const int s0 = decide_par(a, row, P, dl, hist);
+            const int s0 = decide_par<UNAL>(a, row, P, dl, hist);
             if (tid == 0) dl.dl.sh[7] = s0;
         }
         __syncthreads();
@@ -977,7 +1013,7 @@ __global__ void __launch_bounds__(ND) k_decide(PartArgs a, open::OpenArgs o) {
         if (s0 == DS_SCAN) {
             float bv = -INFINITY;
             int bi = -1;
-            row_visit(a, row, P, dl, [&](float w, int id) {
+            row_visit<UNAL>(a, row, P, dl, [&](float w, int id) {
                 if (w == w) best_combine(bv, bi, w, id);
             });
             block_best(bv, bi, dl);
@@ -1055,7 +1091,7 @@ __global__ void __launch_bounds__(ND) k_decide(PartArgs a, open::OpenArgs o) {
         if (!greedy && have) cp = cert_part(maxw, dl.psum[lane], dl.pterm[lane], inv_t, msc, thr);
         const double lo = wave_sum_d(cp.lo), hi = wave_sum_d(cp.hi);
         // window size: exact when every part lies wholly in or wholly out of it
-        const int plen = have ? min(a.part_len, a.vocab - lane * a.part_len) : 0;
+        const int plen = have ? part_count<UNAL>(a, row, lane) : 0;
         const uint32_t pmn = have ? dl.pmin[lane] : 0xFFFFFFFFu;
         const bool out_j = !(maxw * inv_t >= thr);
         const bool in_j = have && pmn != 0xFFFFFFFFu && key2f(pmn) * inv_t >= thr;
@@ -1110,7 +1146,7 @@ __global__ void __launch_bounds__(ND) k_decide(PartArgs a, open::OpenArgs o) {
         if (anyovf) {
             bv = -INFINITY;
             bi = -1;
-            row_visit(a, row, P, dl, [&](float w, int id) {
+            row_visit<UNAL>(a, row, P, dl, [&](float w, int id) {
                 if (w == w) best_combine(bv, bi, w, id);
             });
         }
@@ -1173,10 +1209,11 @@ __global__ void __launch_bounds__(ND) k_decide(PartArgs a, open::OpenArgs o) {
 }
 
 // The second pass and the decision of the rows k_decide<true> left (qs_open.h).
+template <bool UNAL>
 __global__ void __launch_bounds__(ND) k_open(PartArgs a, open::OpenArgs o) {
     __shared__ __align__(16) unsigned char lds[OPEN_LDS];
     const int part = (int)blockIdx.x / a.n_rows, row = (int)blockIdx.x - part * a.n_rows;
-    open::open_select(a, o, row, part, *(open::OpenLds *)lds, *(DecLds *)lds, c_tab_part);
+    open::open_select<UNAL>(a, o, row, part, *(open::OpenLds *)lds, *(DecLds *)lds, c_tab_part);
 }
 
 }  // namespace
@@ -1184,6 +1221,11 @@ __global__ void __launch_bounds__(ND) k_open(PartArgs a, open::OpenArgs o) {
 bool qs_open_row(const qs_row_param &p, int n_vocab) { return open::open_row(p, n_vocab); }
 
 int qs_part_parts(int n_vocab) { return (n_vocab + PART_MAX - 1) / PART_MAX; }
+
+int qs_part_takes(int n_rows, int n_vocab, const void *logits) {
+    return n_rows >= 1 && n_vocab >= 4 && ((uintptr_t)logits % 4) == 0 &&
+           qs_part_parts(n_vocab + 3) <= QS_PART_MAX_PARTS;      // (a row's shift: up to 3)
+}
 
 int qs_part_supported(int n_rows, int n_vocab, int64_t row_stride, const void *logits) {
     if (n_rows < 1 || n_vocab < 4 || n_vocab % 4 != 0 || row_stride % 4 != 0 ||
@@ -1196,7 +1238,7 @@ int qs_part_resident(void) {
     int dev = 0, ncu = 0, nb = 0;
     if (hipGetDevice(&dev) != hipSuccess ||
         hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess ||
-        hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, k_part<false>, NT, 0) != hipSuccess ||
+        hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, k_part<false, false>, NT, 0) != hipSuccess ||
         nb < 1)
         return 0;
     return ncu * nb;
@@ -1211,7 +1253,9 @@ int qs_part_launch(const float *logits, int64_t row_stride, int n_rows, int n_vo
     a.stride = row_stride;
     a.vocab = n_vocab;
     a.n_rows = n_rows;
-    a.parts = qs_part_parts(n_vocab);
+    // 16-byte aligned rows, or rows at any alignment (positions masked at their two ends)
+    const bool unal = !qs_part_supported(n_rows, n_vocab, row_stride, logits);
+    a.parts = qs_part_parts(unal ? n_vocab + 3 : n_vocab);
     a.part_len = PART_MAX;              // whole float4 rows: only a row's last part is short
     a.xcd_map = n_rows >= 8 ? 1 : 0;
     a.st = st;
@@ -1250,30 +1294,28 @@ int qs_part_launch(const float *logits, int64_t row_stride, int n_rows, int n_vo
     if (grid < 1) grid = 1;
     // every row greedy, with the scratch for it: each row decided by its last part
     const bool gf = all_greedy && sc.gbest != nullptr;
-    if (gf)
-        hipLaunchKernelGGL(k_part<true>, dim3((unsigned)grid), dim3(NT), 0, stream, sa,
-                           sa.logits, sa.prm, sa.ring, sa.hlen, sa.hhead, sa.rec, sa.cand);
-    else
-        hipLaunchKernelGGL(k_part<false>, dim3((unsigned)grid), dim3(NT), 0, stream, sa,
-                           sa.logits, sa.prm, sa.ring, sa.hlen, sa.hhead, sa.rec, sa.cand);
+    const dim3 parts_grid((unsigned)grid);
+    hipLaunchKernelGGL(gf ? (unal ? k_part<true, true> : k_part<true, false>)
+                          : (unal ? k_part<false, true> : k_part<false, false>),
+                       parts_grid, dim3(NT), 0, stream, sa, sa.logits, sa.prm, sa.ring, sa.hlen,
+                       sa.hhead, sa.rec, sa.cand);
     hipError_t e = hipGetLastError();
     if (e == hipSuccess && mid) e = hipEventRecord(mid, stream);
     if (e == hipSuccess && !gf) {
         open::OpenArgs oa{};
+        unsigned np = 0;                  // workgroups beside the decisions
         if (open) {
             oa.s = *open;
             oa.parts = qs_open_parts(n_vocab);
-            const unsigned np = (unsigned)(n_rows * oa.parts);
-            hipLaunchKernelGGL(k_decide<true>, dim3((unsigned)n_rows + np), dim3(ND), 0, stream,
+            np = (unsigned)(n_rows * oa.parts);
+        }
+        hipLaunchKernelGGL(open ? (unal ? k_decide<true, true> : k_decide<true, false>)
+                                : (unal ? k_decide<false, true> : k_decide<false, false>),
+                           dim3((unsigned)n_rows + np), dim3(ND), 0, stream, a, oa);
+        e = hipGetLastError();
+        if (e == hipSuccess && open) {
+            hipLaunchKernelGGL(unal ? k_open<true> : k_open<false>, dim3(np), dim3(ND), 0, stream,
                                a, oa);
-            e = hipGetLastError();
-            if (e == hipSuccess) {
-                hipLaunchKernelGGL(k_open, dim3(np), dim3(ND), 0, stream, a, oa);
-                e = hipGetLastError();
-            }
-        } else {
-            hipLaunchKernelGGL(k_decide<false>, dim3((unsigned)n_rows), dim3(ND), 0, stream, a,
-                               oa);
             e = hipGetLastError();
         }
     }

@@ -727,7 +727,7 @@ __global__ void __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(4)
         if (cflag) {                              // a list overflowed: scan the row
             bv = -INFINITY;
             bi = -1;
-            row_visit(a, row, P, dl, [&](float w, int id) {
+            row_visit<false>(a, row, P, dl, [&](float w, int id) {
                 if (w == w) best_combine(bv, bi, w, id);
             });
             block_best(bv, bi, dl);
