@@ -163,6 +163,13 @@ int qs_batch_pick(qs_batch *b, const float *d_logits, int64_t row_stride, int n_
 int qs_batch_pick_rows(qs_batch *b, int row0, const float *d_logits, int64_t row_stride,
                        int n_rows, int n_vocab, int32_t *d_out, qs_pick_diag *d_diag);
 
+/* qs_batch_pick with the ids wanted on the host: enqueues the pick, waits for everything on
+ * the batch's stream and stores the n_rows ids in `ids` (host memory).  Returns what
+ * qs_batch_pick and then qs_batch_synchronize would; on QS_EAGAIN the ids are stored (-3
+ * for the rows to pick again). */
+int qs_batch_pick_ids(qs_batch *b, const float *d_logits, int64_t row_stride, int n_rows,
+                      int n_vocab, int32_t *ids);
+
 /* Which kernels qs_batch_pick uses.  AUTO (the default) takes the row kernel for batches
  * of at least a quarter of a row per CU whose sampling rows have a top-k of at most 256 (or top-k
  * off), the streaming kernels for smaller batches, larger top-k and rows at any other

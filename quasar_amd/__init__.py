@@ -275,11 +275,14 @@ class Batch:
 
     def pick(self, logits_ptr, row_stride, n_rows, n_vocab, diag=False):
         """Pick rows [0, n_rows); returns ids (and a list of PickDiag when diag)."""
+        if not diag:
+            ids = np.empty(max(0, n_rows), dtype=np.int32)
+            check(self._lib.qs_batch_pick_ids(self._b, logits_ptr, row_stride, n_rows, n_vocab,
+                                              ids.ctypes.data), "qs_batch_pick_ids")
+            return ids
         self.pick_async(logits_ptr, row_stride, n_rows, n_vocab, diag)
         self.synchronize()
         ids = self._out.download(np.int32, n_rows)
-        if not diag:
-            return ids
         raw = self._diag.download(np.uint8, C.sizeof(PickDiag) * n_rows)
         d = (PickDiag * n_rows).from_buffer_copy(raw.tobytes())
         return ids, list(d)

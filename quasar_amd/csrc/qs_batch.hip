@@ -542,17 +542,6 @@ __global__ void __launch_bounds__(WG) k_copy_buf(const float4 *x, float4 *y, int
     }
 }
 
-// A one-row pick's result for the host: its id and the batch's error flag stored by one
-// thread into pinned host memory (h: the device's address of it), in place of two
-// device-to-host copies.
-__global__ void __launch_bounds__(64) k_result1(const int32_t *out, const int32_t *err,
-                                                int32_t *h) {
-    if (threadIdx.x == 0) {
-        h[0] = out[0];
-        h[1] = err[0];
-    }
-}
-
 // The kernels' expf, element by element.  Inside [-33, 0] the pipelined kernel's 4-wide
 // window variant (qs_expf4_window, extended table) runs too, and a result different from
 // qs_expf_tab's is reported as NaN, so the comparison with the host C library covers both.
@@ -640,7 +629,10 @@ struct qs_batch {
     void *d_open = nullptr;                // its one allocation
     bool open_dirty = false;               // a launch failed between its two kernels: its
                                            // counters are cleared before the next pick
-    int32_t *h_pin = nullptr;              // pinned: a one-row pick's id and error flag
+    // Pinned host memory the kernels write: the error flag, then a pick's ids (max_rows).
+    // The host reads both after its one wait on the stream, with no copy back: a blocking
+    // 4-byte copy costs about 13 us, and a pick of 32 rows needed two.
+    int32_t *h_pin = nullptr;
     int32_t *d_pin = nullptr;              // the device's address of h_pin
 };
 
@@ -650,7 +642,7 @@ static void batch_release(qs_batch *b) {
     void *ptrs[] = {b->d_prm, b->d_rng, b->d_ring, b->d_hlen, b->d_hhead, b->sc.smax,
                     b->sc.bestv, b->sc.besti, b->sc.sth, b->sc.ckey, b->sc.cid, b->sc.ccnt,
                     b->sc.crej, b->sc.cflag, b->sc.psum, b->sc.pcnt, b->sc.locks,
-                    b->sc.full_keys, b->sc.full_bm, b->sc.err, b->sc.wrec,
+                    b->sc.full_keys, b->sc.full_bm, b->sc.wrec,
                     b->sc.pcand, b->sc.gbest, b->sc.gmaxk, b->sc.gcnt, b->d_hrec,
                     b->d_hbits, b->d_open};
     for (void *p : ptrs)
@@ -710,12 +702,22 @@ static int batch_alloc(qs_batch *b) {
     if (!rc) rc = dev_alloc(&b->sc.locks, b->sc.nslots, "locks");
     if (!rc) rc = dev_alloc(&b->sc.full_keys, (size_t)b->sc.nslots * 2 * V, "full_keys");
     if (!rc) rc = dev_alloc(&b->sc.full_bm, (size_t)b->sc.nslots * (V / 32 + 1), "full_bm");
-    if (!rc) rc = dev_alloc(&b->sc.err, 1, "err");
+    if (!rc) {
+        const size_t n = sizeof(int32_t) * (1 + (size_t)R);
+        hipError_t e = hipHostMalloc((void **)&b->h_pin, n, hipHostMallocDefault);
+        if (e == hipSuccess) {
+            std::memset(b->h_pin, 0, n);
+            e = hipHostGetDevicePointer((void **)&b->d_pin, b->h_pin, 0);
+        } else {
+            b->h_pin = nullptr;
+        }
+        if (e != hipSuccess) rc = hip_fail(e, "pinned ids");
+        b->sc.err = b->d_pin;
+    }
     if (!rc) rc = dev_alloc(&b->sc.gbest, R, "greedy bests");
     if (!rc) rc = dev_alloc(&b->sc.gmaxk, R, "greedy maxima");
     if (!rc) rc = dev_alloc(&b->sc.gcnt, R, "greedy part counts");
     if (!rc && hipMemset(b->sc.locks, 0, sizeof(int32_t) * b->sc.nslots) != hipSuccess) rc = QS_EDEVICE;
-    if (!rc && hipMemset(b->sc.err, 0, sizeof(int32_t)) != hipSuccess) rc = QS_EDEVICE;
     if (!rc && hipMemset(b->sc.gbest, 0, sizeof(uint64_t) * R) != hipSuccess) rc = QS_EDEVICE;
     if (!rc && hipMemset(b->sc.gmaxk, 0, sizeof(uint32_t) * R) != hipSuccess) rc = QS_EDEVICE;
     if (!rc && hipMemset(b->sc.gcnt, 0, sizeof(uint32_t) * R) != hipSuccess) rc = QS_EDEVICE;
@@ -1072,52 +1074,40 @@ int qs_batch_set_mode(qs_batch *b, int mode) {
     return 0;
 }
 
+// The error flag of the picks waited for: QS_EAGAIN (and the flag cleared) when it is set.
+static int take_error(qs_batch *b) {
+    const int32_t err = *(volatile int32_t *)b->h_pin;
+    if (!err) return 0;
+    *(volatile int32_t *)b->h_pin = 0;
+    qs_set_error("a whole-window scratch slot was not free in time (flags %d): the rows "
+                 "involved returned -3 and kept their generator state and history; "
+                 "pick them again", err);
+    return QS_EAGAIN;
+}
+
 int qs_batch_synchronize(qs_batch *b) {
     if (!b) return QS_EINVAL;
     HIP_TRY(hipStreamSynchronize(b->stream), "qs_batch_synchronize");
-    int32_t err = 0;
-    HIP_TRY(hipMemcpy(&err, b->sc.err, sizeof err, hipMemcpyDeviceToHost), "error flag");
-    if (err) {
-        const int32_t zero = 0;
-        (void)hipMemcpy(b->sc.err, &zero, sizeof zero, hipMemcpyHostToDevice);
-        qs_set_error("a whole-window scratch slot was not free in time (flags %d): the rows "
-                     "involved returned -3 and kept their generator state and history; "
-                     "pick them again", err);
-        return QS_EAGAIN;
-    }
-    return 0;
+    return take_error(b);
+}
+
+int qs_batch_pick_ids(qs_batch *b, const float *d_logits, int64_t row_stride, int n_rows,
+                      int n_vocab, int32_t *ids) {
+    if (!b || !ids) { qs_set_error("qs_batch_pick_ids: null argument"); return QS_EINVAL; }
+    if (const int rc = qs_batch_pick(b, d_logits, row_stride, n_rows, n_vocab, b->d_pin + 1,
+                                     nullptr))
+        return rc;
+    HIP_TRY(hipStreamSynchronize(b->stream), "qs_batch_pick_ids");
+    std::memcpy(ids, b->h_pin + 1, sizeof(int32_t) * (size_t)n_rows);
+    return take_error(b);
 }
 
 int qs_batch_pick1_host(qs_batch *b, float *d_logits, const float *logits, int n_vocab,
                         int32_t *d_out, int32_t *id) {
     if (!b || !d_logits || !logits || !d_out || !id) return QS_EINVAL;
-    if (!b->h_pin) {
-        HIP_TRY(hipHostMalloc((void **)&b->h_pin, 2 * sizeof(int32_t), hipHostMallocDefault),
-                "pinned id buffer");
-        if (hipHostGetDevicePointer((void **)&b->d_pin, b->h_pin, 0) != hipSuccess) {
-            (void)hipHostFree(b->h_pin);
-            b->h_pin = nullptr;
-            b->d_pin = nullptr;
-            qs_set_error("pinned id buffer: no device address");
-            return QS_EDEVICE;
-        }
-    }
     HIP_TRY(hipMemcpyAsync(d_logits, logits, sizeof(float) * (size_t)n_vocab,
                            hipMemcpyHostToDevice, b->stream), "logits to the device");
-    if (const int rc = qs_batch_pick(b, d_logits, n_vocab, 1, n_vocab, d_out, nullptr)) return rc;
-    hipLaunchKernelGGL(k_result1, dim3(1), dim3(64), 0, b->stream, d_out, b->sc.err, b->d_pin);
-    HIP_TRY(hipGetLastError(), "k_result1 launch");
-    HIP_TRY(hipStreamSynchronize(b->stream), "one-row pick");
-    if (b->h_pin[1]) {
-        const int32_t zero = 0;
-        (void)hipMemcpy(b->sc.err, &zero, sizeof zero, hipMemcpyHostToDevice);
-        qs_set_error("a whole-window scratch slot was not free in time (flags %d): the row "
-                     "returned -3 and kept its generator state and history; pick it again",
-                     b->h_pin[1]);
-        return QS_EAGAIN;
-    }
-    *id = b->h_pin[0];
-    return 0;
+    return qs_batch_pick_ids(b, d_logits, n_vocab, 1, n_vocab, id);
 }
 
 void *qs_batch_stream(qs_batch *b) { return b ? (void *)b->stream : nullptr; }

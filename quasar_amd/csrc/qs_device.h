@@ -1027,7 +1027,8 @@ __device__ __forceinline__ void full_row(const float *x, int V, int row, const q
     __syncthreads();
     if (slot < 0) {
         if (tid == 0) {
-            atomicOr(sc.err, 1);
+            // (a system-scope store: a batch's flag is in pinned host memory)
+            __hip_atomic_store(sc.err, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
             out[row] = -3;
         }
         return;
