@@ -1195,10 +1195,8 @@ int qs_batch_head_logits(qs_batch *b, const void *d_hidden, const void *d_weight
     if (const int rc = head_check(b, d_hidden, d_weight, n_embd, n_rows, n_vocab, d_logits,
                                   false))
         return rc;
-    RowState st{b->d_prm, b->d_rng, b->d_ring, b->d_hlen, b->d_hhead,
-                b->max_last_n > 0 ? b->max_last_n : 1};
-    return qs_head_launch(d_hidden, d_weight, n_embd, n_rows, n_vocab, d_logits, st, b->sc,
-                          nullptr, nullptr, nullptr, nullptr, b->stream);
+    return qs_logits_launch(d_hidden, d_weight, n_embd, n_rows, n_vocab, d_logits, b->n_cu,
+                            b->stream);
 }
 
 int qs_batch_pick_head(qs_batch *b, const void *d_hidden, const void *d_weight, int n_embd,

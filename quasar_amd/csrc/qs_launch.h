@@ -148,6 +148,10 @@ size_t qs_head_packed_elems(int n_embd, int n_vocab);
 // output-layer kernel reads (qs_head_packed_elems elements at d_packed).
 int qs_head_pack_launch(const void *d_weight, int n_embd, int n_vocab, void *d_packed,
                         hipStream_t stream);
+// Enqueue on `stream`: logits = hidden . weight^T alone (qs_logits.hip) into
+// d_logits[n_rows][n_vocab], one workgroup for each of `n_cu` CUs.
+int qs_logits_launch(const void *d_hidden, const void *d_weight, int n_embd, int n_rows,
+                     int n_vocab, float *d_logits, int n_cu, hipStream_t stream);
 // Enqueue on `stream`: logits = hidden . weight^T (bf16 [n_rows][n_embd] and the packed
 // [n_vocab][n_embd] matrix, fp32 accumulation) into d_logits[n_rows][n_vocab]; with `out`, also
 // the pick of every row from them (rec: n_rows x ceil(n_vocab / QS_HEAD_TILE) records,
