@@ -149,7 +149,8 @@ size_t qs_head_packed_elems(int n_embd, int n_vocab);
 int qs_head_pack_launch(const void *d_weight, int n_embd, int n_vocab, void *d_packed,
                         hipStream_t stream);
 // Enqueue on `stream`: logits = hidden . weight^T alone (qs_logits.hip) into
-// d_logits[n_rows][n_vocab], one workgroup for each of `n_cu` CUs.
+// d_logits[n_rows][n_vocab], one workgroup for each of `n_cu` CUs (n_vocab above
+// QS_HEAD_TILE x n_cu).
 int qs_logits_launch(const void *d_hidden, const void *d_weight, int n_embd, int n_rows,
                      int n_vocab, float *d_logits, int n_cu, hipStream_t stream);
 // Enqueue on `stream`: logits = hidden . weight^T (bf16 [n_rows][n_embd] and the packed

@@ -4,22 +4,31 @@
 //
 // What bounds it: W (2 V E bytes) is read from HBM once and the logits (4 V rows) are written
 // once; at 256 rows x 2048 x 151,936 that is 622 + 156 MB against 159 GFLOP, so the layer
-// streams.  W reaches the CUs at (bytes in flight) / (load latency), and every CU has to
-// stream until the end.  Hence:
+// streams.  W reaches the CUs at (bytes in flight) / (load latency), the CUs have to stream
+// until the end, and what the products cost beside the stream shows.  Hence:
 //
-//   * One workgroup of 8 wavefronts per CU, all of a CU's 160 KB of LDS: a ring of H stages
-//     (from the XCD's L2, short latency) three deep and a ring of W stages (HBM) seven to
-//     nine deep.  Loads return in order per wavefront, so the two rings belong to different
-//     wavefronts: 0-3 load H, 4-7 load W, each waits for its own, and the stage's barrier
-//     joins them.  Six or more W stages of 16 KB stay in flight a CU; the earlier shape (two
-//     workgroups a CU, three shared stages) held 32 KB.
+//   * One workgroup of 8 wavefronts per CU with nearly all of its 160 KB of LDS: a ring of
+//     H stages (from the XCD's L2, short latency) and a ring of W stages (HBM) of 20 KB.
+//     Loads return in order per wavefront, so the two rings belong to different wavefronts:
+//     0-3 load H, 4-7 load W, each waits for its own, and the stage's barrier joins them.  60
+//     to 120 KB of W are in flight a CU; one 128-column tile a workgroup, two of them a CU
+//     with three shared stages (qs_head.hip's shape), held 32.
 //   * The vocabulary is dealt out in 32-column blocks, an equal run for each workgroup (18 or
-//     19 blocks at V = 151,936 on 256 CUs).  One 128-column tile per workgroup made 1,187
-//     workgroups for 512 places: a third round with two thirds of the chip idle.
-//   * A run is cut into tiles of at most 8 blocks whose stages follow each other in the rings
-//     without a break: while a tile's accumulators are stored, the next tile's loads are in
-//     flight.  The stores go straight from the accumulators (32 lanes, 128 consecutive bytes
-//     a row), with no LDS and no barrier.
+//     19 blocks at V = 151,936 on 256 CUs).  Tiles of 128 columns made 1,187 workgroups for
+//     512 places: a third round with two thirds of the chip idle.
+//   * A run is cut into tiles of at most 10 blocks (H is staged again for each: 0.5 GB through
+//     L2 at 256 rows, against 1.2 GB for tiles of 128 columns; 8 blocks: 210 us against 192
+//     at this point of the work) whose stages follow each other in the rings without a break:
+//     while a tile's accumulators are stored, the next tile's loads are in flight.  The
+//     stores go straight from the accumulators (32 lanes, 128 consecutive bytes a row).
+//   * A stage issues a fixed number of loads whose addresses are one scalar offset away from
+//     the last stage's (buffer loads; what lies outside reads nothing), so a stage costs no
+//     address arithmetic and no branches: 192 -> 170 us.
+//
+// Measured, the layer alone in bursts, before (qs_head.hip's kernels) -> now: 256 rows x 2048
+// x 151,936 240 -> 170 us (4.6 TB/s), 128 rows 165 -> 129, 64 rows 138 -> 114, 32 rows 122 ->
+// 105, 1 row 108 -> 93 (6.7 TB/s); 256 x 4096 x 75,968 262 -> 157.  Two halves of the
+// wavefronts alternating reads and products behind four barriers a stage: 231.
 //
 // One stage is 32 embedding elements; the sums run over k in steps of 16 in ascending order,
 // the order of qs_head.hip's fused kernels, so both write the same logits.
@@ -42,6 +51,7 @@ constexpr int LNT = 512;                // threads: 8 wavefronts
 
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef float f32x16 __attribute__((ext_vector_type(16)));
+typedef __attribute__((address_space(3))) void lds_void;
 typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
 
 struct LinArgs {
@@ -55,15 +65,15 @@ struct LinArgs {
 // wavefronts) of a tile of at most TB 32-column blocks; HS and WS ring slots.
 template <int RB> struct LinShape;
 template <> struct LinShape<256> { static constexpr int WRB = 2, RG = 4, CG = 2, TB = 10, HS = 3, WS = 5; };
-template <> struct LinShape<128> { static constexpr int WRB = 2, RG = 2, CG = 4, TB = 10, HS = 3, WS = 6; };
-template <> struct LinShape<64> { static constexpr int WRB = 2, RG = 1, CG = 8, TB = 10, HS = 3, WS = 7; };
-template <> struct LinShape<32> { static constexpr int WRB = 1, RG = 1, CG = 8, TB = 10, HS = 3, WS = 7; };
+template <> struct LinShape<128> { static constexpr int WRB = 2, RG = 2, CG = 4, TB = 10, HS = 4, WS = 6; };
+template <> struct LinShape<64> { static constexpr int WRB = 2, RG = 1, CG = 8, TB = 10, HS = 5, WS = 7; };
+template <> struct LinShape<32> { static constexpr int WRB = 1, RG = 1, CG = 8, TB = 10, HS = 5, WS = 7; };
 
 // 64 bytes a row or column, its four 16-byte segments stored in the order
 // seg ^ ((row / 4) % 4): the lanes of an operand read hit distinct banks.
 template <int RB>
 struct LinLds {
-    uint16_t h[LinShape<RB>::HS][RB][LK];
+    uint16_t h[LinShape<RB>::HS][RB < 64 ? 64 : RB][LK];   // (4 wavefronts x 16 rows at least)
     uint16_t w[LinShape<RB>::WS][LinShape<RB>::TB * 32][LK];
 };
 static_assert(sizeof(LinLds<256>) <= 160 * 1024 && sizeof(LinLds<128>) <= 160 * 1024 &&
@@ -76,19 +86,14 @@ __device__ __forceinline__ void vm_wait() {
     asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
 }
 
-// The same for a count known at run time: N stages of c loads each, 1 <= c <= 5 (uniform).
-template <int N>
-__device__ __forceinline__ void vm_wait_stages(int c) {
-    switch (c) {
-    case 1: vm_wait<N>(); break;
-    case 2: vm_wait<2 * N>(); break;
-    case 3: vm_wait<3 * N>(); break;
-    case 4: vm_wait<4 * N>(); break;
-    default: vm_wait<5 * N>(); break;
-    }
+// A barrier without __syncthreads()'s fence, which would wait for every load in flight; the
+// wavefront's LDS reads are done before it.
+__device__ __forceinline__ void lin_barrier() {
+    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
 }
 
-template <int RB>
+// NT: W by nontemporal loads.
+template <int RB, bool NT>
 __device__ __forceinline__ void lin_run(const LinArgs &a) {
     using S = LinShape<RB>;
     constexpr int WRB = S::WRB, RG = S::RG, CG = S::CG, TB = S::TB, HS = S::HS, WS = S::WS;
@@ -106,55 +111,58 @@ __device__ __forceinline__ void lin_run(const LinArgs &a) {
     const int b1 = (int)((int64_t)a.nblk * (blockIdx.x + 1) / gridDim.x);
     const int nbk = b1 - b0, ntile = (nbk + TB - 1) / TB;
     if (nbk <= 0) return;
-    const int total = ntile * nst;                  // stages of the run
     // tile t of the run: blocks [tile_begin(t), tile_begin(t + 1))
     const int per = nbk / ntile, extra = nbk - per * ntile;
     auto tile_begin = [&](int t) { return b0 + per * t + min(t, extra); };
-    const int wc = (per + 1) / 2;                   // W pieces of a wavefront per stage, at
-                                                    // least (its tiles hold per or per + 1)
 
     const bool wload = wv >= 4;                     // this wavefront loads W (else H)
-    const bool hload = !wload && wv < HPIECES;
-    // the load side: the next stage's tile and stage within it, its ring slot, and where the
-    // wavefront's pieces of the tile start (one per lane: H; uniform: W)
+    // The load side: the next stage's tile and stage within it, its ring slot, and each piece's
+    // byte offset in the wavefront's operand.  Every stage issues the same number of loads, so
+    // the waits are constants: pieces past the tile's columns or the batch's rows, and all of
+    // them past the run's last stage, lie past the operand's buffer and read no memory.
+    constexpr int NL = WL > HL ? WL : HL;
+    constexpr uint32_t NONE = 0xFFFFFFF0u;
+    const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc(
+        wload ? (void *)a.w : (void *)a.h, 0,
+        wload ? (int)((uint32_t)((V + LT - 1) / LT) * (uint32_t)E * (2 * LT)) : B * E * 2,
+        0x00020000);                                // raw buffer, 32-bit data format
     int lt = 0, ls = 0, lslot = 0;
-    uint32_t hoff[HL];                              // bytes
-    uint32_t woff[WL];                              // KB (a packed piece is 1 KB)
-#pragma unroll
-    for (int i = 0; i < HL; ++i) {                  // rows 16 p .. + 16; rows past the batch
-        const int r = (wv + 4 * i) * 16 + (lane >> 2);   // read row 0 (never used)
-        hoff[i] = 2u * (uint32_t)((r < B ? r : 0) * E + ((lane & 3) ^ ((r >> 2) & 3)) * 8);
-    }
-    int lc = 0;                                     // W pieces it loads per stage of the tile
+    uint32_t off[NL];
     auto load_tile = [&]() {
-        // piece p: 16 columns (1 KB, packed contiguously and already swizzled); the last
-        // wavefronts' surplus pieces of an odd share read piece 0 again (cached)
-        const int tb = tile_begin(lt), nb = tile_begin(lt + 1) - tb;
-        lc = (nb + 1) / 2;
+        const int tb = tile_begin(lt), nb = lt < ntile ? tile_begin(lt + 1) - tb : 0;
 #pragma unroll
-        for (int i = 0; i < WL; ++i) {
+        for (int i = 0; i < NL; ++i) {
             const int p = (wv & 3) + 4 * i;
-            const int col = tb * 32 + (p < 2 * nb ? p * 16 : 0);
-            woff[i] = (uint32_t)__builtin_amdgcn_readfirstlane(col / LT * nst * 8 + col % LT / 16);
+            if (wload) {                            // 16 columns, 1 KB, already swizzled
+                const int col = tb * 32 + p * 16;
+                off[i] = p < 2 * nb ? (uint32_t)(col / LT * nst * 8 + col % LT / 16) * 1024u +
+                                          (uint32_t)lane * 16u
+                                    : NONE;
+            } else {                                // rows 16 p .. + 16
+                const int r = p * 16 + (lane >> 2);
+                off[i] = r < B && p < HPIECES && lt < ntile
+                             ? 2u * (uint32_t)(r * E + ((lane & 3) ^ ((r >> 2) & 3)) * 8)
+                             : NONE;
+            }
         }
     };
     load_tile();
-    auto issue = [&]() {
+    auto issue = [&]() __attribute__((always_inline)) {
         if (wload) {
+            uint16_t *dst = &L.w[lslot][(wv & 3) * 16][0];
+            const int at = ls * (LT * LK * 2);
 #pragma unroll
-            for (int i = 0; i < WL; ++i) {
-                if (i >= lc) break;                 // (uniform)
-                __builtin_amdgcn_global_load_lds(
-                    (const char *)a.w + ((uint64_t)(woff[i] + (uint32_t)ls * 8u) << 10) +
-                        (uint32_t)(lane * 16),
-                    &L.w[lslot][((wv & 3) + 4 * i) * 16][0], 16, 0, 2);
-            }
+            for (int i = 0; i < WL; ++i)
+                __builtin_amdgcn_raw_ptr_buffer_load_lds(rs, (lds_void *)(dst + i * 64 * LK), 16,
+                                                         (int)off[i], at, 0, NT ? 2 : 0);
             lslot = lslot + 1 == WS ? 0 : lslot + 1;
-        } else if (hload) {
+        } else {
+            uint16_t *dst = &L.h[lslot][(wv & 3) * 16][0];
+            const int at = ls * (LK * 2);
 #pragma unroll
             for (int i = 0; i < HL; ++i)
-                __builtin_amdgcn_global_load_lds((const char *)(a.h + ls * LK) + hoff[i],
-                                                 &L.h[lslot][(wv + 4 * i) * 16][0], 16, 0, 0);
+                __builtin_amdgcn_raw_ptr_buffer_load_lds(rs, (lds_void *)(dst + i * 64 * LK), 16,
+                                                         (int)off[i], at, 0, 0);
             lslot = lslot + 1 == HS ? 0 : lslot + 1;
         }
         if (++ls == nst) {
@@ -163,13 +171,12 @@ __device__ __forceinline__ void lin_run(const LinArgs &a) {
             load_tile();
         }
     };
-    const int depth = wload ? WS - 1 : HS - 1;      // stages in flight ahead of the products
-    for (int g = 0; g < depth && g < total; ++g) issue();
+    for (int g = 0; g < (wload ? WS : HS) - 1; ++g) issue();
 
     // wavefront w: rows 32 WRB (w % RG) .. + 32 WRB; blocks w / RG + CG j of a tile
     const int rg = wv % RG, cg = wv / RG;
     const int rr = lane & 31, swz = (rr >> 2) & 3;
-    int g = 0, hslot = 0, wslot = 0;
+    int hslot = 0, wslot = 0;
     auto tile = [&](auto nbc, int tb) __attribute__((always_inline)) {
         constexpr int NBW = decltype(nbc)::value;   // this wavefront's blocks
         f32x16 acc[WRB][NBW > 0 ? NBW : 1];
@@ -177,55 +184,55 @@ __device__ __forceinline__ void lin_run(const LinArgs &a) {
         for (int i = 0; i < WRB; ++i)
 #pragma unroll
             for (int j = 0; j < NBW; ++j) acc[i][j] = f32x16{};
-        for (int st = 0; st < nst; ++st, ++g) {
-            // this stage's own loads are in (the later stages' stay in flight; stores of an
-            // earlier tile among them only make the wait longer)
-            if (g + depth < total + 1) {
-                if (wload) vm_wait_stages<WS - 2>(wc);
-                else vm_wait<(HS - 2) * HL>();
-            } else {
-                vm_wait<0>();
-            }
-            // the slots refilled next were read before this barrier by every wavefront
-            asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
-            if (g + depth < total) issue();
-            const uint16_t(*hs)[LK] = L.h[hslot];
-            const uint16_t(*ws)[LK] = L.w[wslot];
-            hslot = hslot + 1 == HS ? 0 : hslot + 1;
-            wslot = wslot + 1 == WS ? 0 : wslot + 1;
+        u32x4 ha[2][WRB], wb[2][NBW > 0 ? NBW : 1];
+        auto read = [&](int ks) __attribute__((always_inline)) {
+            const int sg = ((ks * 2 + (lane >> 5)) ^ swz) * 8;
             if constexpr (NBW > 0) {
 #pragma unroll
-                for (int ks = 0; ks < LK / 16; ++ks) {
-                    const int sg = ((ks * 2 + (lane >> 5)) ^ swz) * 8;
-                    u32x4 ha[WRB], wb[NBW];
+                for (int i = 0; i < WRB; ++i)
+                    ha[ks][i] = *(const u32x4 *)&L.h[hslot][(rg * WRB + i) * 32 + rr][sg];
 #pragma unroll
-                    for (int i = 0; i < WRB; ++i)
-                        ha[i] = *(const u32x4 *)&hs[(rg * WRB + i) * 32 + rr][sg];
-#pragma unroll
-                    for (int j = 0; j < NBW; ++j)
-                        wb[j] = *(const u32x4 *)&ws[(cg + CG * j) * 32 + rr][sg];
-#pragma unroll
-                    for (int j = 0; j < NBW; ++j)
-#pragma unroll
-                        for (int i = 0; i < WRB; ++i)
-                            acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
-                                __builtin_bit_cast(bf16x8, ha[i]),
-                                __builtin_bit_cast(bf16x8, wb[j]), acc[i][j], 0, 0, 0);
-                }
+                for (int j = 0; j < NBW; ++j)
+                    wb[ks][j] = *(const u32x4 *)&L.w[wslot][(cg + CG * j) * 32 + rr][sg];
             }
+        };
+        auto multiply = [&](int ks) __attribute__((always_inline)) {
+#pragma unroll
+            for (int j = 0; j < NBW; ++j)
+#pragma unroll
+                for (int i = 0; i < WRB; ++i)
+                    acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
+                        __builtin_bit_cast(bf16x8, ha[ks][i]), __builtin_bit_cast(bf16x8, wb[ks][j]),
+                        acc[i][j], 0, 0, 0);
+        };
+        for (int st = 0; st < nst; ++st) {
+            // this stage's own loads are in (the later stages' stay in flight; stores of an
+            // earlier tile among them only make the wait longer)
+            if (wload) vm_wait<(WS - 2) * WL>();
+            else vm_wait<(HS - 2) * HL>();
+            // the slots refilled next were read before this barrier by every wavefront
+            lin_barrier();
+            read(0);
+            read(1);
+            issue();
+            multiply(0);
+            multiply(1);
+            hslot = hslot + 1 == HS ? 0 : hslot + 1;
+            wslot = wslot + 1 == WS ? 0 : wslot + 1;
         }
-        // lane l, element q of an accumulator: row (q / 4) * 8 + (l / 32) * 4 + q % 4 of the
-        // block, column l % 32
+        int r0 = rg * WRB * 32 + (lane >> 5) * 4;
+        asm volatile("" : "+v"(r0));                // (its row addresses are formed here, not
+                                                    // held through the products)
 #pragma unroll
         for (int j = 0; j < NBW; ++j) {
             const int col = (tb + cg + CG * j) * 32 + rr;
+            float *out = a.logits + (int64_t)r0 * V + col;
 #pragma unroll
             for (int i = 0; i < WRB; ++i) {
-                const int r0 = (rg * WRB + i) * 32 + (lane >> 5) * 4;
 #pragma unroll
                 for (int q = 0; q < 16; ++q) {
-                    const int r = r0 + (q >> 2) * 8 + (q & 3);
-                    if (r < B && col < V) a.logits[(int64_t)r * V + col] = acc[i][j][q];
+                    const int dr = i * 32 + (q >> 2) * 8 + (q & 3);
+                    if (r0 + dr < B && col < V) out[(int64_t)dr * V] = acc[i][j][q];
                 }
             }
         }
@@ -244,17 +251,28 @@ __device__ __forceinline__ void lin_run(const LinArgs &a) {
         if (mine == 1) tile(std::integral_constant<int, 1>{}, tb);
         if (mine == 0) tile(std::integral_constant<int, 0>{}, tb);
     }
+    vm_wait<0>();                                   // nothing may land in the LDS after the end
 }
 
 // One kernel per shape (a template kernel's host stub is not emitted here).
-__global__ void __launch_bounds__(LNT) __attribute__((amdgpu_waves_per_eu(2, 2)))
-k_logits32(LinArgs a) { lin_run<32>(a); }
-__global__ void __launch_bounds__(LNT) __attribute__((amdgpu_waves_per_eu(2, 2)))
-k_logits64(LinArgs a) { lin_run<64>(a); }
-__global__ void __launch_bounds__(LNT) __attribute__((amdgpu_waves_per_eu(2, 2)))
-k_logits128(LinArgs a) { lin_run<128>(a); }
-__global__ void __launch_bounds__(LNT) __attribute__((amdgpu_waves_per_eu(2, 2)))
-k_logits256(LinArgs a) { lin_run<256>(a); }
+#define LIN_KERNEL(RB)                                                                        \
+    __global__ void __launch_bounds__(LNT) __attribute__((amdgpu_waves_per_eu(2, 2)))         \
+    k_logits##RB(LinArgs a) { lin_run<RB, false>(a); }                                        \
+    __global__ void __launch_bounds__(LNT) __attribute__((amdgpu_waves_per_eu(2, 2)))         \
+    k_logits##RB##_nt(LinArgs a) { lin_run<RB, true>(a); }
+LIN_KERNEL(32)
+LIN_KERNEL(64)
+LIN_KERNEL(128)
+LIN_KERNEL(256)
+#undef LIN_KERNEL
+
+// W is read nontemporally where it and the logits together pass the last-level cache (256 MB):
+// there W would only push out the logits, which the pick reads next (16 rows x 2048: 51.6
+// against 58.0 us at 328 MB of weights, 64 rows: 113.6 against 131.8 at 622 MB; 256 rows x 512
+// x 151,936, 156 + 156 MB: 70 against 72).  What fits stays in it from one step to the next
+// (128 rows x 512 x 151,936, 156 + 78 MB: 41.5 against 46.8 us; 256 x 1024 x 80,000, 164 + 82
+// MB: 58 against 64; at 205 + 3 MB the two are even).
+constexpr uint64_t NT_BYTES = 256ull << 20;
 
 }  // namespace
 
@@ -268,13 +286,14 @@ int qs_logits_launch(const void *d_hidden, const void *d_weight, int n_embd, int
     a.V = n_vocab;
     a.nblk = (n_vocab + 31) / 32;
     a.logits = d_logits;
-    const unsigned grid = (unsigned)(a.nblk < n_cu ? a.nblk : n_cu);
+    const unsigned grid = (unsigned)n_cu;             // (n_vocab > 128 n_cu)
     // the smallest row capacity that holds the batch (the H stages take less of the LDS)
-    hipLaunchKernelGGL(n_rows <= 32    ? k_logits32
-                       : n_rows <= 64  ? k_logits64
-                       : n_rows <= 128 ? k_logits128
-                                       : k_logits256,
-                       dim3(grid), dim3(LNT), 0, stream, a);
+    const bool nt = (2ull * (uint64_t)n_embd + 4ull * (uint64_t)n_rows) * (uint64_t)n_vocab > NT_BYTES;
+    auto *k = n_rows <= 32    ? (nt ? k_logits32_nt : k_logits32)
+              : n_rows <= 64  ? (nt ? k_logits64_nt : k_logits64)
+              : n_rows <= 128 ? (nt ? k_logits128_nt : k_logits128)
+                              : (nt ? k_logits256_nt : k_logits256);
+    hipLaunchKernelGGL(k, dim3(grid), dim3(LNT), 0, stream, a);
     const hipError_t e = hipGetLastError();
     if (e != hipSuccess) {
         qs_set_error("output layer launch: %s", hipGetErrorString(e));
