@@ -71,12 +71,13 @@ int qs_part_resident(void);
 // every row is greedy (`all_greedy`) and sc.gbest is set, each row is decided by its last
 // part in the streaming kernel and the decision kernel is not launched.  With `open` (some
 // row passes qs_open_row; the scratch for n_rows rows), rows the certified decision leaves
-// undecided take the whole-window decision over several workgroups.
+// undecided take the whole-window decision over several workgroups.  The streaming kernel
+// clears the first `clear_locks` words from sc.locks on.
 int qs_part_launch(const float *logits, int64_t row_stride, int n_rows, int n_vocab,
                    const qs::RowState &st, const qs::Scratch &sc, int32_t *out,
                    qs_pick_diag *diag, int resident, hipStream_t stream,
                    hipEvent_t mid = nullptr, bool all_greedy = false,
-                   const OpenScratch *open = nullptr);
+                   const OpenScratch *open = nullptr, int clear_locks = 0);
 
 // ---- the row kernel (qs_row.hip) ----
 

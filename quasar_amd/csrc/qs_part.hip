@@ -102,6 +102,8 @@ struct StreamArgs {
     uint32_t *gmaxk, *gcnt;
     int32_t *ring_w, *hlen_w, *hhead_w, *out;
     qs_pick_diag *diag;
+    int32_t *clear;                  // words the first workgroup sets to 0 (n_clear of them)
+    int n_clear;
 };
 
 constexpr int PART_BM = bitmap_words(PART_MAX);
@@ -563,6 +565,7 @@ k_part(StreamArgs sa, const float *__restrict__ logits, const qs_row_param *__re
     a.hhead = hhead;
     a.rec = rec;
     a.cand = cand;
+    if (blockIdx.x == 0 && tix() < a.n_clear) a.clear[tix()] = 0;
     const Run run = my_run(a);
     if (run.begin >= run.end) return;
     // Every staging load batch of a part after the first goes out right behind that part's
@@ -1247,7 +1250,7 @@ int qs_part_resident(void) {
 int qs_part_launch(const float *logits, int64_t row_stride, int n_rows, int n_vocab,
                    const RowState &st, const Scratch &sc, int32_t *out, qs_pick_diag *diag,
                    int resident, hipStream_t stream, hipEvent_t mid, bool all_greedy,
-                   const OpenScratch *open) {
+                   const OpenScratch *open, int clear_locks) {
     PartArgs a;
     a.logits = logits;
     a.stride = row_stride;
@@ -1285,6 +1288,8 @@ int qs_part_launch(const float *logits, int64_t row_stride, int n_rows, int n_vo
     sa.hhead_w = st.hhead;
     sa.out = out;
     sa.diag = diag;
+    sa.clear = sc.locks;
+    sa.n_clear = clear_locks;
     // a persistent grid: the resident workgroups (a multiple of 8 for the XCD mapping), or
     // one per part when there are fewer parts
     const int64_t total = (int64_t)n_rows * a.parts;
