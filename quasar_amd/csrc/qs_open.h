@@ -27,8 +27,9 @@
 // 151,936 logits, most of them an inv not settled) takes full_row, as every such row did.
 // The histogram only chooses the bins: its error can cost a retry, never a result.
 //
-// Measured (8 rows of N(0, 2) x 151,936 logits, a pick with its ids on the host): 87 us
-// without cuts and 80 us at top-p 0.9, against 18.7 and 12.1 ms in one workgroup a row.
+// Measured (8 rows of N(0, 2) x 151,936 logits, a pick with its ids on the host): 49 us
+// without cuts and 53 us at top-p 0.9, against 18.7 and 12.1 ms in one workgroup a row (with
+// the logits and lists requested only when first needed, 59 us without cuts).
 // Bounds: 8 rows x 151,936 logits are 4.9 MB, read from the last-level cache; the two
 // passes are instruction-bound (an expf a logit each) at about 300 workgroups, and the end
 // is a chain of block steps in one workgroup a row.
@@ -100,19 +101,24 @@ __device__ __forceinline__ int open_bin(float x, float scale) {
     return (int)fminf(fmaxf(b, 0.0f), (float)(ONB - 1));
 }
 
-// Visit the part's logits in the window: f(k, id, x) for this thread's k-th (all threads;
-// the history bitmap in L.bm).  The loads go out before the bitmap is built.
-template <typename F>
-__device__ __forceinline__ void open_visit(const PartArgs &a, int row, const qs_row_param &P,
-                                           int part, float msc, OpenLds &L, F &&f) {
-    const int tid = threadIdx.x, lo = part * OP, hi = min(lo + OP, a.vocab);
+// The part's logits, one load each (what does not depend on them runs under their latency).
+__device__ __forceinline__ void open_load(const PartArgs &a, int row, int part, float (&w)[OQ]) {
+    const int lo = part * OP, hi = min(lo + OP, a.vocab);
     const float *x = a.logits + (int64_t)row * a.stride;
-    float w[OQ];
 #pragma unroll
     for (int k = 0; k < OQ; ++k) {
-        const int i = lo + k * ND + tid;
+        const int i = lo + k * ND + (int)threadIdx.x;
         w[k] = i < hi ? x[i] : -INFINITY;
     }
+}
+
+// Visit the part's loaded logits in the window: f(k, id, x) for this thread's k-th (all
+// threads; the history bitmap in L.bm).
+template <typename F>
+__device__ __forceinline__ void open_visit(const PartArgs &a, int row, const qs_row_param &P,
+                                           int part, float msc, OpenLds &L, float (&w)[OQ],
+                                           F &&f) {
+    const int tid = threadIdx.x, lo = part * OP, hi = min(lo + OP, a.vocab);
     const float rp = P.repeat_penalty, inv_t = P.inv_t, thr = msc - 30.0f;
     // (uniform from the parameters alone: a decision beside the first pass may change the
     // history's length, and build_bitmap's barriers need every thread)
@@ -145,6 +151,8 @@ __device__ __forceinline__ void open_sum(const PartArgs &a, const OpenArgs &o, i
     const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
     const qs_row_param P = row_param(a.st, row);
     if (!open_row(P, a.vocab)) return;
+    float w[OQ];
+    open_load(a, row, part, w);
     if (tid < QS_EXPF_TAB_N) L.tab[tid] = ctab[tid];
     for (int j = tid; j < ONB; j += ND) L.hist[j] = 0ull;
     // the row's largest and least penalised logits from the streaming kernel's records
@@ -177,7 +185,7 @@ __device__ __forceinline__ void open_sum(const PartArgs &a, const OpenArgs &o, i
     const float mp_in = P.min_p * (1.0f + 0x1p-20f), mp_out = P.min_p * (1.0f - 0x1p-20f);
     double acc = 0.0, m_in = 0.0, m_out = 0.0;
     int cnt = 0;
-    open_visit(a, row, P, part, msc, L, [&](int, int, float x) {
+    open_visit(a, row, P, part, msc, L, w, [&](int, int, float x) {
         const float e = qs_expf_core(x, L.tab);
         acc += (double)e;
         ++cnt;
@@ -311,9 +319,19 @@ __device__ __forceinline__ void list_cross(OpenLds &L, int cnt, double base, int
     __syncthreads();
 }
 
-// The list of a row that other workgroups stored, into LDS (all threads).
-__device__ __forceinline__ void load_list(OpenLds &L, const uint64_t *src, int cnt) {
-    for (int j = threadIdx.x; j < cnt; j += ND) L.list[j] = ld_dev(src + j);
+// A row's list that other workgroups stored: its first OPRE entries a thread requested into
+// registers (before the count is known), then all cnt of them into LDS (all threads).
+constexpr int OPRE = 4;
+__device__ __forceinline__ void ask_list(const uint64_t *src, uint64_t (&pre)[OPRE]) {
+#pragma unroll
+    for (int k = 0; k < OPRE; ++k) pre[k] = ld_dev(src + k * ND + threadIdx.x);
+}
+__device__ __forceinline__ void load_list(OpenLds &L, const uint64_t *src,
+                                          const uint64_t (&pre)[OPRE], int cnt) {
+#pragma unroll
+    for (int k = 0; k < OPRE; ++k)
+        if (k * ND + (int)threadIdx.x < cnt) L.list[k * ND + threadIdx.x] = pre[k];
+    for (int j = OPRE * ND + threadIdx.x; j < cnt; j += ND) L.list[j] = ld_dev(src + j);
     __syncthreads();
 }
 
@@ -343,9 +361,12 @@ __device__ __forceinline__ bool open_finish(const PartArgs &a, const OpenArgs &o
                                             float maxl, float msc, uint64_t rs, double u,
                                             int reason, OpenLds &L) {
     const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
+    // one round of requests: the counts, the parts' sums and the head of both lists
     const uint64_t cnts = ld_dev(&o.s.ctl[row].cnt);
-    const int cnt1 = (int)(uint32_t)cnts, cnt2 = (int)(uint32_t)(cnts >> 32);
-    if (cnt1 > OLCAP || cnt2 > OLCAP) return false;
+    const uint64_t *lists = o.s.list + (int64_t)row * 2 * OLCAP;
+    uint64_t pre1[OPRE], pre2[OPRE];
+    if (P.top_p < 1.0f) ask_list(lists, pre1);
+    ask_list(lists + OLCAP, pre2);
     // the parts' sums, in a fixed order
     uint64_t v[8] = {};
     if (tid < o.parts) {
@@ -355,6 +376,8 @@ __device__ __forceinline__ bool open_finish(const PartArgs &a, const OpenArgs &o
     } else {
         v[6] = v[7] = 0xFFFFFFFFull;                  // (min, max) pairs: none
     }
+    const int cnt1 = (int)(uint32_t)cnts, cnt2 = (int)(uint32_t)(cnts >> 32);
+    if (cnt1 > OLCAP || cnt2 > OLCAP) return false;
     double sums[4];
 #pragma unroll
     for (int j = 0; j < 4; ++j) sums[j] = wave_sum_d(__longlong_as_double((long long)v[j]));
@@ -391,14 +414,13 @@ __device__ __forceinline__ bool open_finish(const PartArgs &a, const OpenArgs &o
     }
     __syncthreads();
     const double eps = 8.0 * (double)nwin * 0x1p-53;
-    const uint64_t *lists = o.s.list + (int64_t)row * 2 * OLCAP;
     // sample.c:155-160: the shortest prefix whose running sum reaches top_p
     int n_topp = nwin;
     double rsum = all;
     if (P.top_p < 1.0f) {
         const double tp = (double)P.top_p;
         if (!(all * (1.0 + eps) < tp)) {
-            load_list(L, lists, cnt1);
+            load_list(L, lists, pre1, cnt1);
             list_cross(L, cnt1, a1, above1, min1, max1, tp, eps);
             if (!L.cross.ok) return false;
             n_topp = L.cross.pos + 1;
@@ -416,7 +438,7 @@ __device__ __forceinline__ bool open_finish(const PartArgs &a, const OpenArgs &o
         }
     }
     const double r = u * rsum;                        // sample.c:170-175
-    load_list(L, lists + OLCAP, cnt2);
+    load_list(L, lists + OLCAP, pre2, cnt2);
     list_cross(L, cnt2, a2, above2, min2, max2, r, eps);
     if (!L.cross.ok || L.cross.pos >= n) return false;
     if (tid == 0) {
@@ -462,6 +484,8 @@ __device__ __forceinline__ void open_select(const PartArgs &a, const OpenArgs &o
     uint64_t *ghist = o.s.hist + (int64_t)row * ONB;
     const qs_row_param P = row_param(a.st, row);
     if (!open_row(P, a.vocab)) return;
+    float w[OQ];
+    open_load(a, row, part, w);
     const int reason = ctl->reason;
     if (reason == 0) {                                // decided: the histogram back to zero
         if (part == 0)
@@ -543,7 +567,7 @@ __device__ __forceinline__ void open_select(const PartArgs &a, const OpenArgs &o
         float p[OQ];
 #pragma unroll
         for (int k = 0; k < OQ; ++k) p[k] = 0.0f;
-        open_visit(a, row, P, part, msc, L, [&](int k, int, float x) {
+        open_visit(a, row, P, part, msc, L, w, [&](int k, int, float x) {
             const float pk = qs_expf_core(x, L.tab) * inv;
             const uint32_t pb = __float_as_uint(pk);
             const double pd = (double)pk;
