@@ -99,12 +99,12 @@ __device__ __forceinline__ int part_count(const PartArgs &a, int row, int j) {
     return max(hi - lo, 0);
 }
 
-// Visit the row's penalised logits (f(w, id) on every thread's share; all threads): in
-// blocks of XBM logits, each with its history bitmap in LDS, read XUP float4s per thread at
+// Visit the penalised logits at positions [from, to) of the row (from a multiple of 4; f(w, id)
+// on every thread's share; all threads): in blocks of XBM logits, each with its history bitmap in LDS, read XUP float4s per thread at
 // a time with every load issued before the first is used.  UNAL: rows at any alignment.
 template <bool UNAL, typename F>
-__device__ __forceinline__ void row_visit(const PartArgs &a, int row, const qs_row_param &P,
-                                          DecLds &dl, F &&f) {
+__device__ __forceinline__ void range_visit(const PartArgs &a, int row, const qs_row_param &P,
+                                            DecLds &dl, int from, int to, F &&f) {
     const int tid = threadIdx.x;
     const float rp = P.repeat_penalty;
     const int cap = P.ring_cap;                   // (clamped: row_param)
@@ -112,9 +112,9 @@ __device__ __forceinline__ void row_visit(const PartArgs &a, int row, const qs_r
     ring_pos(a.st, row, cap, len, head);
     const bool pen = rp > 1.0f && len > 0 && cap > 0;
     const int32_t *ring = a.st.ring + (int64_t)row * a.st.ring_stride;
-    const int sh = UNAL ? row_shift(a.logits, a.stride, row) : 0, end = a.vocab + sh;
+    const int sh = UNAL ? row_shift(a.logits, a.stride, row) : 0, end = min(to, a.vocab + sh);
     const float4 *x4 = (const float4 *)(a.logits + (int64_t)row * a.stride - sh);
-    for (int lo = 0; lo < end; lo += XBM) {
+    for (int lo = from; lo < end; lo += XBM) {
         const int hi = min(lo + XBM, end), c_hi = UNAL ? (hi + 3) >> 2 : hi >> 2;
         if (pen) {                                    // sample.c:118-120: each id once
             for (int j = tid; j < bitmap_words(XBM); j += ND) dl.bm[j] = 0u;
@@ -150,6 +150,12 @@ __device__ __forceinline__ void row_visit(const PartArgs &a, int row, const qs_r
         }
         if (pen) __syncthreads();                     // the block's bitmap is read
     }
+}
+
+template <bool UNAL, typename F>
+__device__ __forceinline__ void row_visit(const PartArgs &a, int row, const qs_row_param &P,
+                                          DecLds &dl, F &&f) {
+    range_visit<UNAL>(a, row, P, dl, 0, a.vocab + 3, f);   // (the row's end bounds it)
 }
 
 // The row's exact softmax denominator and window size (sample.c:136-149), recomputed from

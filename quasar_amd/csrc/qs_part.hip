@@ -953,6 +953,95 @@ __device__ __forceinline__ int decide_par(const PartArgs &a, int row, const qs_r
                          hist);
 }
 
+// Whether widening the row's candidates can decide it: the cuts read past the proven prefix
+// and fewer than top-k + 2 candidates lie above the row's bound (the bound is the key below a
+// candidate's, so the last one is never proved).
+__device__ __forceinline__ bool widen_pays(int why, const qs_row_param &P, const CertTotals &t) {
+    return (why == CF_PREFIX || why == CF_TOPP_PAST || why == CF_MINP_PAST ||
+            why == CF_KEEP_PAST) &&
+           P.top_k > 0 && t.total < row_ksel(P) + 2 && !t.cflag;
+}
+
+// The row's bound is the largest part bound, and a part's bound is the least of its eight
+// wavefronts' maxima: now and then (about one row in 300 at top-k 40 and 10 parts) one lies so
+// high that fewer than top-k + 2 logits of the row exceed it, and such a row went to the exact
+// path, 170 us for its one workgroup.  Here the WIDEN parts with the largest bounds are read
+// again for their logits in (r2, r1], r1 the row's bound and r2 the largest bound of the other
+// parts; with the other parts' candidates there (complete above r2) the row's bound becomes
+// r2.  All threads; dl.ct and the candidates are updated; false (dl.ct as it was) where the
+// bound cannot fall or the candidates do not fit.
+constexpr int WIDEN = 3;
+template <bool UNAL>
+__device__ __forceinline__ bool widen(const PartArgs &a, int row, const qs_row_param &P,
+                                      DecLds &dl) {
+    const int tid = threadIdx.x;
+    // the WIDEN largest bounds (descending) and their parts, then r2
+    uint32_t r[WIDEN + 1];
+    int p[WIDEN + 1];
+#pragma unroll
+    for (int i = 0; i <= WIDEN; ++i) {
+        r[i] = 0u;
+        p[i] = -1;
+    }
+    for (int j = 0; j < a.parts; ++j) {
+        uint32_t v = dl.prej[j];
+        int q = j;
+#pragma unroll
+        for (int i = 0; i <= WIDEN; ++i)
+            if (v > r[i] || p[i] < 0) {
+                const uint32_t tv = r[i];
+                const int tq = p[i];
+                r[i] = v;
+                p[i] = q;
+                v = tv;
+                q = tq;
+            }
+    }
+    const uint32_t r1 = r[0], r2 = p[WIDEN] >= 0 ? r[WIDEN] : 0u;
+    if (!(r2 < r1)) return false;
+    if (tid == 0) dl.gcount = dl.ct.total;
+    __syncthreads();
+    auto take = [&](uint32_t k, int id) {
+        if (k > r2 && k <= r1) {
+            const int at = atomicAdd(&dl.gcount, 1);
+            if (at < FCAP) {
+                dl.keys[at] = k;
+                dl.ids[at] = id;
+            }
+        }
+    };
+    const int NL = a.parts * NWV;
+    const int64_t l0 = (int64_t)row * NL;
+    for (int L = tid; L < NL; L += ND) {
+        const int n = min(a.sc.wrec[l0 + L].cnt, WCAP);
+        for (int i = 0; i < n; ++i) {
+            const uint2 e = a.sc.pcand[(l0 + L) * WCAP + i];
+            take(e.x, (int)e.y);
+        }
+    }
+    static_assert(WIDEN == 3, "the parts below");
+    for (int i = 0; i < WIDEN; ++i) {
+        const int q = i == 0 ? p[0] : i == 1 ? p[1] : p[2];   // (uniform)
+        if (q < 0) break;
+        range_visit<UNAL>(a, row, P, dl, q * a.part_len, (q + 1) * a.part_len,
+                          [&](float w, int id) {
+                              // what the part kept is above its bound and taken from its list
+                              const uint32_t k = w == w ? f2key(w) : 0u;
+                              take(k <= dl.prej[q] ? k : 0u, id);
+                          });
+        __syncthreads();
+    }
+    __syncthreads();
+    const int total = dl.gcount;
+    if (total > FCAP) return false;                   // (the first candidates stand as before)
+    if (tid == 0) {
+        dl.ct.total = total;
+        dl.ct.rej = r2;
+    }
+    __syncthreads();
+    return true;
+}
+
 // The LDS of a workgroup that may take either a row's decision or a part of an open row.
 constexpr size_t OPEN_LDS =
     sizeof(open::OpenLds) > sizeof(DecLds) ? sizeof(open::OpenLds) : sizeof(DecLds);
@@ -960,8 +1049,9 @@ constexpr size_t OPEN_LDS =
 // The row decisions.  OPEN: some row has no top-k and the scratch of qs_open.h is there;
 // rows it serves that the certified decision leaves undecided are left to k_open, and the
 // workgroups past the row decisions take those rows' first pass meanwhile (the chip is
-// otherwise idle: a decision is one workgroup a row).  UNAL: rows at any alignment.
-template <bool OPEN, bool UNAL>
+// otherwise idle: a decision is one workgroup a row).  UNAL: rows at any alignment.  WIDE: rows short of
+// candidates take more (widen).
+template <bool OPEN, bool UNAL, bool WIDE>
 __global__ void __launch_bounds__(ND) k_decide(PartArgs a, open::OpenArgs o) {
     __shared__ __align__(16) unsigned char lds[OPEN ? OPEN_LDS : sizeof(DecLds)];
     DecLds &dl = *(DecLds *)lds;
@@ -1023,11 +1113,28 @@ __global__ void __launch_bounds__(ND) k_decide(PartArgs a, open::OpenArgs o) {
             if (tid == 0) record_greedy(row, P, bv, bi, dl.ct.maxl, x[0], st, a.out, a.diag);
             return;
         }
-        const CertTotals t = dl.ct;
+        CertTotals t = dl.ct;
         int status = s0;
         if (s0 == DS_BLOCK) {
             status = cert_row_block<ND>(row, P, t, dl.keys, dl.ids, dl.srt, dl.dl, st, a.out,
                                         a.diag, hist);
+            if (status == 0) return;
+        }
+        if (WIDE && widen_pays(status, P, t) && widen<UNAL>(a, row, P, dl)) {
+            t = dl.ct;
+            if (row_ksel(P) <= 64 && t.total <= WAVE_CAND) {
+                if (wv == 0) {
+                    const int s1 = cert_row_wave(row, P, t, dl.keys, dl.ids, dl.srt, dl.dl.tab,
+                                                 st, a.out, a.diag, hist);
+                    if (lane == 0) dl.dl.sh[7] = s1;
+                }
+                __syncthreads();
+                status = dl.dl.sh[7];
+                __syncthreads();
+            } else {
+                status = cert_row_block<ND>(row, P, t, dl.keys, dl.ids, dl.srt, dl.dl, st, a.out,
+                                            a.diag, hist);
+            }
             if (status == 0) return;
         }
         undecided(t, status);
@@ -1190,9 +1297,11 @@ __global__ void __launch_bounds__(ND) k_decide(PartArgs a, open::OpenArgs o) {
             }
         });
     }
+    if (tid == 0) dl.ct = t;
     __syncthreads();
     int status = finite ? CF_MSC : CF_INPUT;
-    if (finite && fabsf(t.msc) < CERT_MSC_MAX && t.total <= FCAP) {
+    for (bool first = true; finite && fabsf(t.msc) < CERT_MSC_MAX && t.total <= FCAP;
+         first = false) {
         if (row_ksel(P) <= 64 && t.total <= WAVE_CAND) {
             if (tid < 64) {
                 const int s = cert_row_wave(row, P, t, dl.keys, dl.ids, dl.srt, dl.dl.tab, st,
@@ -1206,8 +1315,13 @@ __global__ void __launch_bounds__(ND) k_decide(PartArgs a, open::OpenArgs o) {
             status = cert_row_block<ND>(row, P, t, dl.keys, dl.ids, dl.srt, dl.dl, st, a.out,
                                         a.diag, hist);
         }
+        if (status == 0) return;
+        if (!WIDE || !first || !widen_pays(status, P, t)) break;
+        __syncthreads();
+        const bool more = widen<UNAL>(a, row, P, dl);
+        t = dl.ct;
+        if (!more) break;
     }
-    if (status == 0) return;
     undecided(t, status);
 }
 
@@ -1314,9 +1428,16 @@ int qs_part_launch(const float *logits, int64_t row_stride, int n_rows, int n_vo
             oa.parts = qs_open_parts(n_vocab);
             np = (unsigned)(n_rows * oa.parts);
         }
-        hipLaunchKernelGGL(open ? (unal ? k_decide<true, true> : k_decide<true, false>)
-                                : (unal ? k_decide<false, true> : k_decide<false, false>),
-                           dim3((unsigned)n_rows + np), dim3(ND), 0, stream, a, oa);
+        // The widening costs every decision about 0.5 us (its registers and code: one row 15.9
+        // against 16.3 us a pick, 32 rows 31.5 against 32.2) and saves a row that needs it 170,
+        // about one in 300 (unaligned 48-row batches: one in seven held such a row), so it
+        // pays from a few rows on.
+        const bool wide = n_rows > 4;
+        auto *k = open   ? (unal ? k_decide<true, true, true> : k_decide<true, false, true>)
+                  : unal ? k_decide<false, true, true>
+                  : wide ? k_decide<false, false, true>
+                         : k_decide<false, false, false>;
+        hipLaunchKernelGGL(k, dim3((unsigned)n_rows + np), dim3(ND), 0, stream, a, oa);
         e = hipGetLastError();
         if (e == hipSuccess && open) {
             hipLaunchKernelGGL(unal ? k_open<true> : k_open<false>, dim3(np), dim3(ND), 0, stream,
