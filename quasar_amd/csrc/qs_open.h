@@ -23,8 +23,9 @@
 // lie within eps = 8 n 2^-53 of these; a position counts only when its sums clear the target
 // by eps on both sides.  The order inside a list is exact, and a position counts only when
 // its p lies strictly between the least p above the list and the largest below it, so no
-// tie reaches across the list's ends.  What is not proved (about one pick in 10^4 at
-// 151,936 logits, most of them an inv not settled) takes full_row, as every such row did.
+// tie reaches across the list's ends.  Where inv is not settled (about one row in 1,000 at
+// 151,936 logits) the sum is taken again in id order; what is not proved (about one row in
+// 50,000, and rows of few values) takes full_row, as every such row did.
 // The histogram only chooses the bins: its error can cost a retry, never a result.
 //
 // Measured (8 rows of N(0, 2) x 151,936 logits, a pick with its ids on the host): 49 us
@@ -474,6 +475,45 @@ __device__ __forceinline__ bool open_finish(const PartArgs &a, const OpenArgs &o
     return true;
 }
 
+// The row's softmax denominator exactly as sample.c:147-149 adds it, by one workgroup: a part's
+// numerators at a time into LDS (0 outside the window, which adds nothing), then one binary64
+// chain over them in id order.  All threads; the sum in every thread.
+__device__ __forceinline__ double open_sum_in_order(const PartArgs &a, const OpenArgs &o, int row,
+                                                    const qs_row_param &P, float msc,
+                                                    OpenLds &L) {
+    static_assert(OLCAP >= OP && OP % 16 == 0, "a part's numerators in the list's LDS");
+    const int tid = threadIdx.x;
+    double *e = (double *)L.list;
+    double acc = 0.0;
+    for (int q = 0; q < o.parts; ++q) {
+        float w[OQ];
+        open_load(a, row, q, w);
+#pragma unroll
+        for (int k = 0; k < OQ; ++k) e[k * ND + tid] = 0.0;
+        open_visit(a, row, P, q, msc, L, w, [&](int k, int, float x) {
+            e[k * ND + tid] = (double)qs_expf_core(x, L.tab);
+        });
+        __syncthreads();
+        if (tid < 64) {                               // (every lane the same chain)
+            const double2 *d = (const double2 *)e;
+            for (int i = 0; i < OP / 2; i += 8) {
+                double2 v[8];
+#pragma unroll
+                for (int j = 0; j < 8; ++j) v[j] = d[i + j];
+#pragma unroll
+                for (int j = 0; j < 8; ++j) {
+                    acc += v[j].x;
+                    acc += v[j].y;
+                }
+            }
+        }
+        __syncthreads();
+    }
+    if (tid == 0) L.rd[4][0] = acc;
+    __syncthreads();
+    return L.rd[4][0];
+}
+
 // The second pass: one part of a row whose decision kernel left it here.
 template <bool UNAL>
 __device__ __forceinline__ void open_select(const PartArgs &a, const OpenArgs &o, int row,
@@ -532,14 +572,14 @@ __device__ __forceinline__ void open_select(const PartArgs &a, const OpenArgs &o
 #pragma unroll
     for (int q = 0; q < 4; ++q) c[q] += cb;
     const bool good = !a.sc.sum_in_order && inv_settled(S, nwin);   // (uniform)
-    const float inv = (float)(1.0 / S);
+    float inv = (float)(1.0 / S);
     uint64_t rs = a.st.rng[row];
     const double u = rng_unit(rs);
-    if (good) {
-        // the bins of the top-p cut, and the sum the draw scales with (histogram units)
-        const bool topp = P.top_p < 1.0f;
+    // the bins of the top-p cut, and the sum the draw scales with (histogram units)
+    const bool topp = P.top_p < 1.0f;
+    int c_lo = ONB, c_hi = ONB, d_lo, d_hi;
+    {
         double r_lo = T, r_hi = T;
-        int c_lo = ONB, c_hi = ONB;
         if (topp) {
             const double m = (double)P.top_p * T;
             first_bins(c, m * (1.0 - BIN_SLACK), m * (1.0 + BIN_SLACK), &L.ru[7][0]);
@@ -557,137 +597,156 @@ __device__ __forceinline__ void open_select(const PartArgs &a, const OpenArgs &o
         }
         first_bins(c, u * r_lo * (1.0 - BIN_SLACK), u * r_hi * (1.0 + BIN_SLACK) + 1.0,
                    &L.ru[7][2]);
-        const int d_lo = (int)L.ru[7][2], d_hi = min((int)L.ru[7][3], ONB - 1);
-        // the part's share: sums above the bins, the entries inside them
-        const float floor_p = P.min_p * inv;
-        double a1 = 0.0, a2 = 0.0, am = 0.0, all = 0.0;
-        int n1 = 0, n2 = 0, nm = 0;
-        uint32_t min1 = 0xFFFFFFFFu, max1 = 0u, min2 = 0xFFFFFFFFu, max2 = 0u;
-        uint32_t in1 = 0u, in2 = 0u;
-        float p[OQ];
+        d_lo = (int)L.ru[7][2];
+        d_hi = min((int)L.ru[7][3], ONB - 1);
+    }
+    // Each part takes its own share.  Where the parts' sum leaves inv open (about one row in
+    // 1,000 at 151,936 logits), the last part adds the row's numerators in id order (1 ms) and
+    // takes every part's share itself (the whole-window sort took 12 to 19 ms).
+    bool all_parts = false;
+    for (int q = part;;) {
+        if (good || all_parts) {
+            // the part's share: sums above the bins, the entries inside them
+            const float floor_p = P.min_p * inv;
+            double a1 = 0.0, a2 = 0.0, am = 0.0, all = 0.0;
+            int n1 = 0, n2 = 0, nm = 0;
+            uint32_t min1 = 0xFFFFFFFFu, max1 = 0u, min2 = 0xFFFFFFFFu, max2 = 0u;
+            uint32_t in1 = 0u, in2 = 0u;
+            float p[OQ];
 #pragma unroll
-        for (int k = 0; k < OQ; ++k) p[k] = 0.0f;
-        open_visit(a, row, P, part, msc, L, w, [&](int k, int, float x) {
-            const float pk = qs_expf_core(x, L.tab) * inv;
-            const uint32_t pb = __float_as_uint(pk);
-            const double pd = (double)pk;
-            const int b = open_bin(x, scale);
-            p[k] = pk;
-            all += pd;
-            if (topp) {
-                if (b < c_lo) {
-                    a1 += pd;
-                    ++n1;
-                    min1 = min(min1, pb);
-                } else if (b <= c_hi) {
-                    in1 |= 1u << k;
+            for (int k = 0; k < OQ; ++k) p[k] = 0.0f;
+            open_visit(a, row, P, q, msc, L, w, [&](int k, int, float x) {
+                const float pk = qs_expf_core(x, L.tab) * inv;
+                const uint32_t pb = __float_as_uint(pk);
+                const double pd = (double)pk;
+                const int b = open_bin(x, scale);
+                p[k] = pk;
+                all += pd;
+                if (topp) {
+                    if (b < c_lo) {
+                        a1 += pd;
+                        ++n1;
+                        min1 = min(min1, pb);
+                    } else if (b <= c_hi) {
+                        in1 |= 1u << k;
+                    } else {
+                        max1 = max(max1, pb);
+                    }
+                }
+                if (b < d_lo) {
+                    a2 += pd;
+                    ++n2;
+                    min2 = min(min2, pb);
+                } else if (b <= d_hi) {
+                    in2 |= 1u << k;
                 } else {
-                    max1 = max(max1, pb);
+                    max2 = max(max2, pb);
+                }
+                if (pk >= floor_p) {
+                    am += pd;
+                    ++nm;
+                }
+            });
+            // the entries' places: one addition to the row's two counts for the workgroup
+            const uint32_t mine = (uint32_t)__popc(in1) | ((uint32_t)__popc(in2) << 16);
+            const uint32_t pre = wave_scan(mine);         // (counts up to 4096: 16 bits each)
+            a1 = wave_sum_d(a1);
+            a2 = wave_sum_d(a2);
+            am = wave_sum_d(am);
+            all = wave_sum_d(all);
+            n1 = wave_sum_i(n1);
+            n2 = wave_sum_i(n2);
+            nm = wave_sum_i(nm);
+            min1 = wave_min_u(min1);
+            max1 = wave_max_u(max1);
+            min2 = wave_min_u(min2);
+            max2 = wave_max_u(max2);
+            __syncthreads();                              // (rd and ru were read above)
+            if (lane == 63) L.ru[7][wv] = pre;
+            if (lane == 0) {
+                L.rd[0][wv] = a1;
+                L.rd[1][wv] = a2;
+                L.rd[2][wv] = am;
+                L.rd[3][wv] = all;
+                L.ru[0][wv] = (uint32_t)n1;
+                L.ru[1][wv] = (uint32_t)n2;
+                L.ru[2][wv] = (uint32_t)nm;
+                L.ru[3][wv] = min1;
+                L.ru[4][wv] = max1;
+                L.ru[5][wv] = min2;
+                L.ru[6][wv] = max2;
+            }
+            __syncthreads();
+            uint32_t off = pre - mine, tot = 0u;
+            for (int j = 0; j < ND / 64; ++j) {
+                if (j < wv) off += L.ru[7][j];
+                tot += L.ru[7][j];
+            }
+            if (tid == 0) {
+                L.base = tot ? add_dev(&ctl->cnt, (uint64_t)(tot & 0xFFFFu) |
+                                                      ((uint64_t)(tot >> 16) << 32))
+                             : 0ull;
+                a1 = a2 = am = all = 0.0;
+                n1 = n2 = nm = 0;
+                min1 = min2 = 0xFFFFFFFFu;
+                max1 = max2 = 0u;
+                for (int j = 0; j < ND / 64; ++j) {
+                    a1 += L.rd[0][j];
+                    a2 += L.rd[1][j];
+                    am += L.rd[2][j];
+                    all += L.rd[3][j];
+                    n1 += (int)L.ru[0][j];
+                    n2 += (int)L.ru[1][j];
+                    nm += (int)L.ru[2][j];
+                    min1 = min(min1, L.ru[3][j]);
+                    max1 = max(max1, L.ru[4][j]);
+                    min2 = min(min2, L.ru[5][j]);
+                    max2 = max(max2, L.ru[6][j]);
+                }
+                uint64_t *dst = (uint64_t *)(o.s.prec + (int64_t)row * o.parts + q);
+                st_dev(dst + 0, (uint64_t)__double_as_longlong(a1));
+                st_dev(dst + 1, (uint64_t)__double_as_longlong(a2));
+                st_dev(dst + 2, (uint64_t)__double_as_longlong(am));
+                st_dev(dst + 3, (uint64_t)__double_as_longlong(all));
+                st_dev(dst + 4, (uint64_t)(uint32_t)n1 | ((uint64_t)(uint32_t)n2 << 32));
+                st_dev(dst + 5, (uint64_t)(uint32_t)nm);
+                st_dev(dst + 6, (uint64_t)min1 | ((uint64_t)max1 << 32));
+                st_dev(dst + 7, (uint64_t)min2 | ((uint64_t)max2 << 32));
+            }
+            __syncthreads();
+            const uint64_t gb = L.base;
+            uint32_t at1 = (uint32_t)gb + (off & 0xFFFFu), at2 = (uint32_t)(gb >> 32) + (off >> 16);
+            uint64_t *lists = o.s.list + (int64_t)row * 2 * OLCAP;
+#pragma unroll
+            for (int k = 0; k < OQ; ++k) {
+                const uint64_t key = pid_key(p[k], q * OP + k * ND + tid);
+                if ((in1 >> k) & 1u) {
+                    if (at1 < OLCAP) st_dev(lists + at1, key);
+                    ++at1;
+                }
+                if ((in2 >> k) & 1u) {
+                    if (at2 < OLCAP) st_dev(lists + OLCAP + at2, key);
+                    ++at2;
                 }
             }
-            if (b < d_lo) {
-                a2 += pd;
-                ++n2;
-                min2 = min(min2, pb);
-            } else if (b <= d_hi) {
-                in2 |= 1u << k;
-            } else {
-                max2 = max(max2, pb);
-            }
-            if (pk >= floor_p) {
-                am += pd;
-                ++nm;
-            }
-        });
-        // the entries' places: one addition to the row's two counts for the workgroup
-        const uint32_t mine = (uint32_t)__popc(in1) | ((uint32_t)__popc(in2) << 16);
-        const uint32_t pre = wave_scan(mine);         // (counts up to 4096: 16 bits each)
-        a1 = wave_sum_d(a1);
-        a2 = wave_sum_d(a2);
-        am = wave_sum_d(am);
-        all = wave_sum_d(all);
-        n1 = wave_sum_i(n1);
-        n2 = wave_sum_i(n2);
-        nm = wave_sum_i(nm);
-        min1 = wave_min_u(min1);
-        max1 = wave_max_u(max1);
-        min2 = wave_min_u(min2);
-        max2 = wave_max_u(max2);
-        __syncthreads();                              // (rd and ru were read above)
-        if (lane == 63) L.ru[7][wv] = pre;
-        if (lane == 0) {
-            L.rd[0][wv] = a1;
-            L.rd[1][wv] = a2;
-            L.rd[2][wv] = am;
-            L.rd[3][wv] = all;
-            L.ru[0][wv] = (uint32_t)n1;
-            L.ru[1][wv] = (uint32_t)n2;
-            L.ru[2][wv] = (uint32_t)nm;
-            L.ru[3][wv] = min1;
-            L.ru[4][wv] = max1;
-            L.ru[5][wv] = min2;
-            L.ru[6][wv] = max2;
         }
+        stores_done();                                // every wavefront's, then counted
         __syncthreads();
-        uint32_t off = pre - mine, tot = 0u;
-        for (int j = 0; j < ND / 64; ++j) {
-            if (j < wv) off += L.ru[7][j];
-            tot += L.ru[7][j];
+        if (all_parts) {
+            if (++q == o.parts) break;
+        } else {
+            if (tid == 0) L.flag = add_dev(&ctl->done, 1) == o.parts - 1;
+            __syncthreads();
+            if (!L.flag) return;
+            if (good) break;
+            S = open_sum_in_order(a, o, row, P, msc, L);
+            inv = (float)(1.0 / S);
+            all_parts = true;
+            q = 0;
         }
-        if (tid == 0) {
-            L.base = tot ? add_dev(&ctl->cnt, (uint64_t)(tot & 0xFFFFu) |
-                                                  ((uint64_t)(tot >> 16) << 32))
-                         : 0ull;
-            a1 = a2 = am = all = 0.0;
-            n1 = n2 = nm = 0;
-            min1 = min2 = 0xFFFFFFFFu;
-            max1 = max2 = 0u;
-            for (int j = 0; j < ND / 64; ++j) {
-                a1 += L.rd[0][j];
-                a2 += L.rd[1][j];
-                am += L.rd[2][j];
-                all += L.rd[3][j];
-                n1 += (int)L.ru[0][j];
-                n2 += (int)L.ru[1][j];
-                nm += (int)L.ru[2][j];
-                min1 = min(min1, L.ru[3][j]);
-                max1 = max(max1, L.ru[4][j]);
-                min2 = min(min2, L.ru[5][j]);
-                max2 = max(max2, L.ru[6][j]);
-            }
-            uint64_t *dst = (uint64_t *)(o.s.prec + (int64_t)row * o.parts + part);
-            st_dev(dst + 0, (uint64_t)__double_as_longlong(a1));
-            st_dev(dst + 1, (uint64_t)__double_as_longlong(a2));
-            st_dev(dst + 2, (uint64_t)__double_as_longlong(am));
-            st_dev(dst + 3, (uint64_t)__double_as_longlong(all));
-            st_dev(dst + 4, (uint64_t)(uint32_t)n1 | ((uint64_t)(uint32_t)n2 << 32));
-            st_dev(dst + 5, (uint64_t)(uint32_t)nm);
-            st_dev(dst + 6, (uint64_t)min1 | ((uint64_t)max1 << 32));
-            st_dev(dst + 7, (uint64_t)min2 | ((uint64_t)max2 << 32));
-        }
-        __syncthreads();
-        const uint64_t gb = L.base;
-        uint32_t at1 = (uint32_t)gb + (off & 0xFFFFu), at2 = (uint32_t)(gb >> 32) + (off >> 16);
-        uint64_t *lists = o.s.list + (int64_t)row * 2 * OLCAP;
-#pragma unroll
-        for (int k = 0; k < OQ; ++k) {
-            const uint64_t key = pid_key(p[k], part * OP + k * ND + tid);
-            if ((in1 >> k) & 1u) {
-                if (at1 < OLCAP) st_dev(lists + at1, key);
-                ++at1;
-            }
-            if ((in2 >> k) & 1u) {
-                if (at2 < OLCAP) st_dev(lists + OLCAP + at2, key);
-                ++at2;
-            }
-        }
+        open_load(a, row, q, w);
     }
-    stores_done();                                    // every wavefront's, then counted
-    __syncthreads();
-    if (tid == 0) L.flag = add_dev(&ctl->done, 1) == o.parts - 1;
-    __syncthreads();
-    if (!L.flag) return;
-    const bool ok = good && open_finish(a, o, row, P, S, inv, nwin, maxl, msc, rs, u, reason, L);
+    const bool ok = open_finish(a, o, row, P, S, inv, nwin, maxl, msc, rs, u, reason, L);
     // every part has read the histogram and the counts: zero for the next pick
     for (int b = tid; b < ONB; b += ND) st_dev(ghist + b, (uint64_t)0);
     if (tid == 0) {

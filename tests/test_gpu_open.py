@@ -74,3 +74,32 @@ def test_open_rows(oracle, V):
         print(V, first, "paths", paths, flush=True)
         b.close()
         buf.free()
+
+
+@pytest.mark.parametrize("V", [4092, 40963, 151936])
+def test_open_rows_summed_in_id_order(oracle, V):
+    """The same rows with the denominator always taken in id order (as where the parts' sum
+    leaves inv open): the row's last part does every part's share, and the sum is the
+    restatement's bit for bit."""
+    import quasar_amd as qa
+    x = rows_of(V, V + 1)[[0, 1, 4, 5]]
+    B = len(x)
+    dev = qa.DeviceBuffer.from_array(x)
+    for cfg in SETTINGS[:4]:
+        b = qa.Batch(B, V, 64)
+        b.set_sum_in_order(1)
+        b.config(0, B, *cfg, seeds=np.arange(7, 7 + B))
+        got = [b.pick(dev.ptr, V, B, V, diag=True) for _ in range(2)]
+        for r in range(B):
+            s = oracle.sampler()
+            s.config(*cfg, seed=7 + r)
+            for k in range(2):
+                want, od = s.pick_diag(x[r])
+                d = got[k][1][r]
+                assert int(got[k][0][r]) == want, (cfg, r, k, d.path)
+                assert d.keep == od["keep"], (cfg, r, k)
+                if d.path == qa.PATH_FULL:
+                    assert d.sum == od["sum"] and d.rank == od["rank"], (cfg, r, k)
+            assert b.get_state(r)[0] == s.rng
+        b.close()
+    dev.free()
