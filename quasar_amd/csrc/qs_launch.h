@@ -149,9 +149,12 @@ size_t qs_head_packed_elems(int n_embd, int n_vocab);
 // output-layer kernel reads (qs_head_packed_elems elements at d_packed).
 int qs_head_pack_launch(const void *d_weight, int n_embd, int n_vocab, void *d_packed,
                         hipStream_t stream);
+// Whether qs_logits_launch can address this layer: a workgroup's run of W and the hidden rows
+// each lie within one buffer (under 4 GiB).  No device of 288 GB holds a layer that does not.
+bool qs_logits_fits(int n_embd, int n_rows, int n_vocab, int n_cu);
 // Enqueue on `stream`: logits = hidden . weight^T alone (qs_logits.hip) into
 // d_logits[n_rows][n_vocab], one workgroup for each of `n_cu` CUs (n_vocab above
-// QS_HEAD_TILE x n_cu).
+// QS_HEAD_TILE x n_cu; qs_logits_fits).
 int qs_logits_launch(const void *d_hidden, const void *d_weight, int n_embd, int n_rows,
                      int n_vocab, float *d_logits, int n_cu, hipStream_t stream);
 // Enqueue on `stream`: logits = hidden . weight^T (bf16 [n_rows][n_embd] and the packed

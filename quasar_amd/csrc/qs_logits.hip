@@ -119,12 +119,17 @@ __device__ __forceinline__ void lin_run(const LinArgs &a) {
     // The load side: the next stage's tile and stage within it, its ring slot, and each piece's
     // byte offset in the wavefront's operand.  Every stage issues the same number of loads, so
     // the waits are constants: pieces past the tile's columns or the batch's rows, and all of
-    // them past the run's last stage, lie past the operand's buffer and read no memory.
+    // them past the run's last stage, lie past the operand's buffer and read no memory.  W's
+    // buffer is the packed tiles of this run, its base formed in 64 bits: W as a whole may pass
+    // the 4 GiB that a buffer's size and offsets hold (256,000 x 12,288 is 6.3 GB), a run does
+    // not (qs_logits_fits).
     constexpr int NL = WL > HL ? WL : HL;
     constexpr uint32_t NONE = 0xFFFFFFF0u;
+    const int t0 = b0 * 32 / LT, t1 = (b1 * 32 + LT - 1) / LT;      // the run's packed tiles
+    const uint16_t *wrun = a.w + (int64_t)t0 * E * LT;
     const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc(
-        wload ? (void *)a.w : (void *)a.h, 0,
-        wload ? (int)((uint32_t)((V + LT - 1) / LT) * (uint32_t)E * (2 * LT)) : B * E * 2,
+        wload ? (void *)wrun : (void *)a.h, 0,
+        (int)(wload ? (uint32_t)(t1 - t0) * (uint32_t)E * (2 * LT) : (uint32_t)B * (uint32_t)E * 2u),
         0x00020000);                                // raw buffer, 32-bit data format
     int lt = 0, ls = 0, lslot = 0;
     uint32_t off[NL];
@@ -135,13 +140,14 @@ __device__ __forceinline__ void lin_run(const LinArgs &a) {
             const int p = (wv & 3) + 4 * i;
             if (wload) {                            // 16 columns, 1 KB, already swizzled
                 const int col = tb * 32 + p * 16;
-                off[i] = p < 2 * nb ? (uint32_t)(col / LT * nst * 8 + col % LT / 16) * 1024u +
-                                          (uint32_t)lane * 16u
+                off[i] = p < 2 * nb ? ((uint32_t)(col / LT - t0) * (uint32_t)(nst * 8) +
+                                       (uint32_t)(col % LT / 16)) * 1024u + (uint32_t)lane * 16u
                                     : NONE;
             } else {                                // rows 16 p .. + 16
                 const int r = p * 16 + (lane >> 2);
                 off[i] = r < B && p < HPIECES && lt < ntile
-                             ? 2u * (uint32_t)(r * E + ((lane & 3) ^ ((r >> 2) & 3)) * 8)
+                             ? 2u * ((uint32_t)r * (uint32_t)E +
+                                     (uint32_t)(((lane & 3) ^ ((r >> 2) & 3)) * 8))
                              : NONE;
             }
         }
@@ -275,6 +281,14 @@ LIN_KERNEL(256)
 constexpr uint64_t NT_BYTES = 256ull << 20;
 
 }  // namespace
+
+bool qs_logits_fits(int n_embd, int n_rows, int n_vocab, int n_cu) {
+    // (a run of ceil(blocks / n_cu) blocks of 32 columns touches at most this many tiles)
+    const int64_t blocks = ((n_vocab + 31) / 32 + n_cu - 1) / n_cu;
+    const int64_t run = (blocks * 32 + LT - 1) / LT + 1;
+    const int64_t w = run * n_embd * (2 * LT), h = (int64_t)n_rows * n_embd * 2;
+    return w < 0xFFFFFFF0ll && h < 0xFFFFFFF0ll;
+}
 
 int qs_logits_launch(const void *d_hidden, const void *d_weight, int n_embd, int n_rows,
                      int n_vocab, float *d_logits, int n_cu, hipStream_t stream) {

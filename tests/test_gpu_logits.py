@@ -38,3 +38,33 @@ def test_logits_of_column_runs(rows, E, V):
     want, mag = hd @ wd.t(), hd.abs() @ wd.abs().t()
     assert ((got.double() - want).abs() <= E * 2.0 ** -24 * mag + 1e-30).all()
     b.close()
+
+
+@pytest.mark.parametrize("rows,E,V", [
+    (3, 8128, 262144), (3, 8192, 262144), (70, 8192, 262144), (5, 12288, 256000)])
+def test_logits_of_matrices_around_4_gib(rows, E, V):
+    """Packed weights a tile row under 2^32 bytes, of 2^32 and of 6.3e9: every column against
+    the fused kernels' logits bit for bit, and columns on both sides of the 2^32nd byte (and
+    the first and the last) against a float64 product within the bound above."""
+    import quasar_amd as qa
+    g = torch.Generator(device="cuda")
+    g.manual_seed(rows + E)
+    h = torch.randn((rows, E), generator=g, device="cuda").bfloat16()
+    w = torch.randn((V, E), generator=g, device="cuda", dtype=torch.bfloat16)
+    packed = torch.empty(qa.head_packed_bytes(E, V), dtype=torch.uint8, device="cuda")
+    got, fused = (torch.full((rows, V), 7.0, device="cuda") for _ in range(2))
+    torch.cuda.synchronize()
+    b = qa.Batch(rows, V, 8)
+    b.config(0, rows, 0.7, 0.95, 40, 0.05, 1.0, 0, seeds=np.arange(1, rows + 1))
+    b.head_pack(w.data_ptr(), E, V, packed.data_ptr())
+    b.head_logits(h.data_ptr(), packed.data_ptr(), E, rows, V, got.data_ptr())
+    b.synchronize()
+    b.pick_head(h.data_ptr(), packed.data_ptr(), E, rows, V, fused.data_ptr())
+    assert torch.equal(got, fused)
+    at = min(2 ** 32 // (2 * E), V)
+    cols = torch.tensor(sorted({c for m in (0, at, V) for c in range(max(0, m - 200), min(V, m + 200))}),
+                        device="cuda")
+    hd, wd = h.double(), w[cols].double()
+    want, mag = hd @ wd.t(), hd.abs() @ wd.abs().t()
+    assert ((got[:, cols].double() - want).abs() <= E * 2.0 ** -24 * mag).all()
+    b.close()
