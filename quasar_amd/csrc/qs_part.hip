@@ -1014,9 +1014,12 @@ __device__ __forceinline__ bool widen(const PartArgs &a, int row, const qs_row_p
     const int64_t l0 = (int64_t)row * NL;
     for (int L = tid; L < NL; L += ND) {
         const int n = min(a.sc.wrec[l0 + L].cnt, WCAP);
+        const uint32_t bound = dl.prej[L / NWV];
         for (int i = 0; i < n; ++i) {
             const uint2 e = a.sc.pcand[(l0 + L) * WCAP + i];
-            take(e.x, (int)e.y);
+            // (a list whose threshold is +0 holds -0 logits too, whose key is the part's bound:
+            // the part's second reading takes those)
+            take(e.x > bound ? e.x : 0u, (int)e.y);
         }
     }
     static_assert(WIDEN == 3, "the parts below");
