@@ -733,13 +733,14 @@ static void open_alloc(qs_batch *b) {
     const size_t P = qs_open_parts(b->max_vocab);
     const size_t hist = sizeof(uint64_t) * QS_OPEN_BINS * R, sum = sizeof(OpenSum) * P * R,
                  prec = sizeof(OpenPartRec) * P * R, list = sizeof(uint64_t) * 2 * QS_OPEN_LIST * R,
-                 ctl = sizeof(OpenCtl) * R;
+                 ctl = sizeof(OpenCtl) * R, queue = sizeof(int32_t) * (1 + R);
+    const size_t bytes = hist + prec + sum + list + ctl + queue;
     uint8_t *p = nullptr;
-    if (hipMalloc((void **)&p, hist + prec + sum + list + ctl) != hipSuccess) {
+    if (hipMalloc((void **)&p, bytes) != hipSuccess) {
         (void)hipGetLastError();
         return;
     }
-    if (hipMemset(p, 0, hist + prec + sum + list + ctl) != hipSuccess) {
+    if (hipMemset(p, 0, bytes) != hipSuccess) {
         (void)hipGetLastError();
         (void)hipFree(p);
         return;
@@ -750,6 +751,7 @@ static void open_alloc(qs_batch *b) {
     b->open.sum = (OpenSum *)(p + hist + prec);
     b->open.list = (uint64_t *)(p + hist + prec + sum);
     b->open.ctl = (OpenCtl *)(p + hist + prec + sum + list);
+    b->open.queue = (int32_t *)(p + hist + prec + sum + list + ctl);
 }
 
 static int upload_rows(qs_batch *b, int row0, int n_rows) {

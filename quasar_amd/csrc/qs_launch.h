@@ -44,6 +44,8 @@ struct OpenCtl {
     float maxl, scale;
 };
 struct OpenScratch {
+    int32_t *queue;                  // a count (zeroed by the streaming kernel), then the rows
+                                     // that the decision kernel left undecided
     uint64_t *hist;                  // [rows][QS_OPEN_BINS]  (null: no such scratch)
     OpenSum *sum;                    // [rows][parts]
     OpenPartRec *prec;               // [rows][parts]

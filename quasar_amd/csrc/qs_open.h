@@ -9,13 +9,18 @@
 // rsum, and the top-p cut the first whose running sum reaches top_p.  Both are found by
 // selection, in two passes over the row split into parts of OP logits:
 //
-//   sums (open_sum, the workgroups of the decision kernel past its row decisions, running
-//     beside them): each part's exact numerators e (the host-libm-equal expf), their
+//   sums (open_sum): each part's exact numerators e (the host-libm-equal expf), their
 //     binary64 sum, and a histogram of their mass over ONB bins of the scaled logit.
 //   select (k_open): inv from the parts' sums; from the histogram the few bins that hold
 //     the top-p cut and the drawn position; each part then adds up p = fl(e * inv) above
 //     those bins and lists the (p, id) inside them.  The row's last part to finish finds
 //     the two positions in the lists.
+//
+// The decision kernel queues the rows it leaves undecided, and k_open takes the queue's.  In
+// picks of few rows the sums are taken by workgroups of the decision kernel past its row
+// decisions, beside them and for every row without a top-k (the chip is otherwise idle); in
+// larger picks that would hold up rows that need none, so a launch of its own (k_open_sum)
+// takes the queue's rows.  An empty queue costs a launch one load.
 //
 // Why it is the reference's result.  inv is proved to be the reference's float (inv_settled).
 // Every p is the reference's float.  Any order of adding n nonnegative binary64 numbers
@@ -62,6 +67,7 @@ static_assert(OP % ND == 0 && ONB == 4 * ND && OSUB == ND && OQ <= 32, "the thre
 struct OpenArgs {
     OpenScratch s;
     int parts;                       // open parts per row
+    int beside;                      // 1: the sums are taken beside the decisions
 };
 
 // The rows this path takes: sampling rows whose top-k cuts nothing.
@@ -76,14 +82,16 @@ struct Cross {
     int ok;
 };
 
-struct OpenLds {
+struct OpenSumLds {                  // what a part's sums need
     uint64_t tab[QS_EXPF_TAB_N];
     uint64_t hist[ONB];              // the part's histogram; later the ranked entries
-    uint64_t list[OLCAP];
-    uint64_t sub[OSUB];
     uint32_t bm[OP / 32];
     double rd[5][ND / 64];
     uint32_t ru[8][ND / 64];
+};
+struct OpenLds : OpenSumLds {
+    uint64_t list[OLCAP];
+    uint64_t sub[OSUB];
     uint64_t base;
     Cross cross;
     int ns, flag;
@@ -117,8 +125,8 @@ __device__ __forceinline__ void open_load(const PartArgs &a, int row, int part, 
 // threads; the history bitmap in L.bm).
 template <typename F>
 __device__ __forceinline__ void open_visit(const PartArgs &a, int row, const qs_row_param &P,
-                                           int part, float msc, OpenLds &L, float (&w)[OQ],
-                                           F &&f) {
+                                           int part, float msc, OpenSumLds &L,
+                                           float (&w)[OQ], F &&f) {
     const int tid = threadIdx.x, lo = part * OP, hi = min(lo + OP, a.vocab);
     const float rp = P.repeat_penalty, inv_t = P.inv_t, thr = msc - 30.0f;
     // (uniform from the parameters alone: a decision beside the first pass may change the
@@ -144,11 +152,11 @@ __device__ __forceinline__ double block_sum_d(double v, double (&r)[ND / 64]) {
     return t;
 }
 
-// One part of the first pass.  Runs beside the row decisions: the decision of its own row
-// may record an id meanwhile, and then nothing here is used (the bitmap reads stay in range
-// whatever the ring holds, and a bin is always inside the histogram).
+// One part of the first pass.  Beside the row decisions the decision of its own row may record
+// an id meanwhile, and then nothing here is used (the bitmap reads stay in range whatever the
+// ring holds, and a bin is always inside the histogram).
 __device__ __forceinline__ void open_sum(const PartArgs &a, const OpenArgs &o, int row, int part,
-                                         OpenLds &L, const uint64_t *ctab) {
+                                         OpenSumLds &L, const uint64_t *ctab) {
     const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
     const qs_row_param P = row_param(a.st, row);
     if (!open_row(P, a.vocab)) return;
@@ -514,7 +522,7 @@ __device__ __forceinline__ double open_sum_in_order(const PartArgs &a, const Ope
     return L.rd[4][0];
 }
 
-// The second pass: one part of a row whose decision kernel left it here.
+// The second pass: one part of a row of the queue.
 template <bool UNAL>
 __device__ __forceinline__ void open_select(const PartArgs &a, const OpenArgs &o, int row,
                                             int part, OpenLds &L, DecLds &dl,
@@ -523,15 +531,9 @@ __device__ __forceinline__ void open_select(const PartArgs &a, const OpenArgs &o
     OpenCtl *ctl = o.s.ctl + row;
     uint64_t *ghist = o.s.hist + (int64_t)row * ONB;
     const qs_row_param P = row_param(a.st, row);
-    if (!open_row(P, a.vocab)) return;
     float w[OQ];
     open_load(a, row, part, w);
     const int reason = ctl->reason;
-    if (reason == 0) {                                // decided: the histogram back to zero
-        if (part == 0)
-            for (int b = tid; b < ONB; b += ND) ghist[b] = 0ull;
-        return;
-    }
     if (tid < QS_EXPF_TAB_N) L.tab[tid] = ctab[tid];
     if (tid < 4) L.ru[7][tid] = ONB;
     const float maxl = ctl->maxl, scale = ctl->scale, msc = maxl * P.inv_t;

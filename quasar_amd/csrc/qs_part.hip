@@ -1045,23 +1045,19 @@ __device__ __forceinline__ bool widen(const PartArgs &a, int row, const qs_row_p
     return true;
 }
 
-// The LDS of a workgroup that may take either a row's decision or a part of an open row.
-constexpr size_t OPEN_LDS =
-    sizeof(open::OpenLds) > sizeof(DecLds) ? sizeof(open::OpenLds) : sizeof(DecLds);
-
 // The row decisions.  OPEN: some row has no top-k and the scratch of qs_open.h is there;
-// rows it serves that the certified decision leaves undecided are left to k_open, and the
-// workgroups past the row decisions take those rows' first pass meanwhile (the chip is
-// otherwise idle: a decision is one workgroup a row).  UNAL: rows at any alignment.  WIDE: rows short of
-// candidates take more (widen).
+// rows it serves that the certified decision leaves undecided are queued for k_open, and
+// workgroups past the row decisions, where there are any, take those rows' first pass
+// meanwhile.  UNAL: rows at any alignment.  WIDE: rows short of candidates take more (widen).
 template <bool OPEN, bool UNAL, bool WIDE>
 __global__ void __launch_bounds__(ND) k_decide(PartArgs a, open::OpenArgs o) {
-    __shared__ __align__(16) unsigned char lds[OPEN ? OPEN_LDS : sizeof(DecLds)];
-    DecLds &dl = *(DecLds *)lds;
+    __shared__ DecLds dl;
     if constexpr (OPEN) {
+        static_assert(sizeof(open::OpenSumLds) <= sizeof(DecLds) &&
+                          alignof(open::OpenSumLds) <= alignof(DecLds), "a part's sums");
         if ((int)blockIdx.x >= a.n_rows) {
             const int i = (int)blockIdx.x - a.n_rows, part = i / a.n_rows;
-            open::open_sum(a, o, i - part * a.n_rows, part, *(open::OpenLds *)lds, c_tab_part);
+            open::open_sum(a, o, i - part * a.n_rows, part, *(open::OpenSumLds *)&dl, c_tab_part);
             return;
         }
     }
@@ -1078,12 +1074,15 @@ __global__ void __launch_bounds__(ND) k_decide(PartArgs a, open::OpenArgs o) {
     if (tid < QS_EXPF_TAB_N) dl.dl.tab[tid] = c_tab_part[tid];
     RowHist hist{0ull, 0, 0};
     if (tid < 64 && !greedy) hist = row_hist(st, row);
-    // a row the certified decision does not cover: left to k_open, or decided here
+    // a row the certified decision does not cover: queued for k_open, or decided here
     if (OPEN && tid == 0) o.s.ctl[row].reason = 0;
     auto undecided = [&](const CertTotals &t, int reason) __attribute__((always_inline)) {
         if constexpr (OPEN) {
             if (open::open_row(P, a.vocab) && isfinite(t.msc)) {
-                if (tid == 0) o.s.ctl[row].reason = reason;
+                if (tid == 0) {
+                    o.s.ctl[row].reason = reason;
+                    o.s.queue[1 + add_dev(o.s.queue, 1)] = row;
+                }
                 return;
             }
         }
@@ -1328,13 +1327,39 @@ __global__ void __launch_bounds__(ND) k_decide(PartArgs a, open::OpenArgs o) {
     undecided(t, status);
 }
 
-// The second pass and the decision of the rows k_decide<true> left (qs_open.h).
+// The passes over the rows that k_decide queued (qs_open.h), a workgroup for each part of every
+// row of the pick; those past the queue leave.  Neighbours take the same part of different
+// rows: their additions go to different histograms and counters.
+template <typename F>
+__device__ __forceinline__ void open_queue(const open::OpenArgs &o, F &&f) {
+    const int n = o.s.queue[0], i = blockIdx.x, part = n ? i / n : o.parts;
+    if (part < o.parts) f(o.s.queue[1 + i - part * n], part);
+}
+__global__ void __launch_bounds__(ND) k_open_sum(PartArgs a, open::OpenArgs o) {
+    __shared__ open::OpenSumLds L;
+    open_queue(o, [&](int row, int part) { open::open_sum(a, o, row, part, L, c_tab_part); });
+}
 template <bool UNAL>
 __global__ void __launch_bounds__(ND) k_open(PartArgs a, open::OpenArgs o) {
-    __shared__ __align__(16) unsigned char lds[OPEN_LDS];
-    const int part = (int)blockIdx.x / a.n_rows, row = (int)blockIdx.x - part * a.n_rows;
-    open::open_select<UNAL>(a, o, row, part, *(open::OpenLds *)lds, *(DecLds *)lds, c_tab_part);
+    constexpr size_t BYTES =
+        sizeof(open::OpenLds) > sizeof(DecLds) ? sizeof(open::OpenLds) : sizeof(DecLds);
+    __shared__ __align__(16) unsigned char lds[BYTES];
+    // a row decided although its sums were taken beside it: its histogram back to zero
+    if (o.beside && (int)blockIdx.x < a.n_rows && o.s.ctl[blockIdx.x].reason == 0)
+        for (int b = threadIdx.x; b < open::ONB; b += ND)
+            o.s.hist[(int64_t)blockIdx.x * open::ONB + b] = 0ull;
+    open_queue(o, [&](int row, int part) {
+        open::open_select<UNAL>(a, o, row, part, *(open::OpenLds *)lds, *(DecLds *)lds, c_tab_part);
+    });
 }
+
+// Up to this many workgroups of the first pass run beside the decisions (20 rows of 151,936);
+// past it they are a launch of their own, over the queue.  Rows without a top-k that the
+// certified decision covers, a pick beside / with the launch / with neither pass (an empty
+// launch is about 2.3 us): 8 rows 23 / - / 20.4 us, 17 rows 26.0 / 26.8 / -, 32 rows 30.2 / 26.7 /
+// 22.1, 60 rows 51 / 34 / 29: most of the first pass's workgroups wait for a place there.  Flat
+// rows lose the overlap: 17 rows 42 / 52 us, 32 rows 55 / 65, 60 rows 88 / 91.
+constexpr unsigned OPEN_BESIDE = 768;
 
 }  // namespace
 
@@ -1405,8 +1430,8 @@ int qs_part_launch(const float *logits, int64_t row_stride, int n_rows, int n_vo
     sa.hhead_w = st.hhead;
     sa.out = out;
     sa.diag = diag;
-    sa.clear = sc.locks;
-    sa.n_clear = clear_locks;
+    sa.clear = open ? open->queue : sc.locks;
+    sa.n_clear = open ? 1 : clear_locks;
     // a persistent grid: the resident workgroups (a multiple of 8 for the XCD mapping), or
     // one per part when there are fewer parts
     const int64_t total = (int64_t)n_rows * a.parts;
@@ -1425,23 +1450,28 @@ int qs_part_launch(const float *logits, int64_t row_stride, int n_rows, int n_vo
     if (e == hipSuccess && mid) e = hipEventRecord(mid, stream);
     if (e == hipSuccess && !gf) {
         open::OpenArgs oa{};
-        unsigned np = 0;                  // workgroups beside the decisions
+        unsigned np = 0, beside = 0;      // workgroups of an open pass, beside the decisions
         if (open) {
             oa.s = *open;
             oa.parts = qs_open_parts(n_vocab);
             np = (unsigned)(n_rows * oa.parts);
+            oa.beside = np <= OPEN_BESIDE;
+            if (oa.beside) beside = np;
         }
         // The widening costs every decision about 0.5 us (its registers and code: one row 15.9
         // against 16.3 us a pick, 32 rows 31.5 against 32.2) and saves a row that needs it 170,
         // about one in 300 (unaligned 48-row batches: one in seven held such a row), so it
         // pays from a few rows on.
         const bool wide = n_rows > 4;
-        auto *k = open   ? (unal ? k_decide<true, true, true> : k_decide<true, false, true>)
-                  : unal ? k_decide<false, true, true>
-                  : wide ? k_decide<false, false, true>
-                         : k_decide<false, false, false>;
-        hipLaunchKernelGGL(k, dim3((unsigned)n_rows + np), dim3(ND), 0, stream, a, oa);
+        auto *k = unal   ? (open ? k_decide<true, true, true> : k_decide<false, true, true>)
+                  : wide ? (open ? k_decide<true, false, true> : k_decide<false, false, true>)
+                         : (open ? k_decide<true, false, false> : k_decide<false, false, false>);
+        hipLaunchKernelGGL(k, dim3((unsigned)n_rows + beside), dim3(ND), 0, stream, a, oa);
         e = hipGetLastError();
+        if (e == hipSuccess && open && !oa.beside) {
+            hipLaunchKernelGGL(k_open_sum, dim3(np), dim3(ND), 0, stream, a, oa);
+            e = hipGetLastError();
+        }
         if (e == hipSuccess && open) {
             hipLaunchKernelGGL(unal ? k_open<true> : k_open<false>, dim3(np), dim3(ND), 0, stream,
                                a, oa);
