@@ -289,6 +289,10 @@ int qs_batch_set_spin_limit(qs_batch *b, int attempts);
  * equals the reference's bit for bit); 0, the default, only where needed. */
 int qs_batch_set_sum_in_order(qs_batch *b, int always);
 
+/* QS_PATH_FULL rows since the batch was made that were decided by selecting the two positions
+ * of their whole window, not by sorting it (a test hook; waits for the batch's stream). */
+int qs_batch_selected_rows(qs_batch *b, int *n);
+
 /* `iters` plain streaming copies of `bytes` (a multiple of 16, 16-byte aligned) from
  * d_src to d_dst, then a device synchronization: a kernel of known memory traffic for
  * calibrating hardware memory counters. */

@@ -310,6 +310,12 @@ class Batch:
         check(self._lib.qs_batch_set_sum_in_order(self._b, int(always)),
               "qs_batch_set_sum_in_order")
 
+    def selected_rows(self):
+        """Whole-window rows decided by selection so far (qs_batch_selected_rows)."""
+        n = C.c_int(0)
+        check(self._lib.qs_batch_selected_rows(self._b, C.byref(n)), "qs_batch_selected_rows")
+        return n.value
+
     def set_spin_limit(self, attempts):
         """Attempts a row makes at a whole-window scratch slot (qs_batch_set_spin_limit)."""
         check(self._lib.qs_batch_set_spin_limit(self._b, int(attempts)),

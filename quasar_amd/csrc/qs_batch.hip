@@ -733,7 +733,7 @@ static void open_alloc(qs_batch *b) {
     const size_t P = qs_open_parts(b->max_vocab);
     const size_t hist = sizeof(uint64_t) * QS_OPEN_BINS * R, sum = sizeof(OpenSum) * P * R,
                  prec = sizeof(OpenPartRec) * P * R, list = sizeof(uint64_t) * 2 * QS_OPEN_LIST * R,
-                 ctl = sizeof(OpenCtl) * R, queue = sizeof(int32_t) * (1 + R);
+                 ctl = sizeof(OpenCtl) * R, queue = sizeof(int32_t) * (2 + R);
     const size_t bytes = hist + prec + sum + list + ctl + queue;
     uint8_t *p = nullptr;
     if (hipMalloc((void **)&p, bytes) != hipSuccess) {
@@ -752,6 +752,7 @@ static void open_alloc(qs_batch *b) {
     b->open.list = (uint64_t *)(p + hist + prec + sum);
     b->open.ctl = (OpenCtl *)(p + hist + prec + sum + list);
     b->open.queue = (int32_t *)(p + hist + prec + sum + list + ctl);
+    b->open.selected = b->open.queue + 1 + R;
 }
 
 static int upload_rows(qs_batch *b, int row0, int n_rows) {
@@ -1113,6 +1114,19 @@ int qs_batch_pick1_host(qs_batch *b, float *d_logits, const float *logits, int n
 }
 
 void *qs_batch_stream(qs_batch *b) { return b ? (void *)b->stream : nullptr; }
+
+int qs_batch_selected_rows(qs_batch *b, int *n) {
+    if (!b || !n) {
+        qs_set_error("qs_batch_selected_rows: bad arguments");
+        return QS_EINVAL;
+    }
+    HIP_TRY(hipStreamSynchronize(b->stream), "qs_batch_selected_rows");
+    *n = 0;
+    if (b->d_open)
+        HIP_TRY(hipMemcpy(n, b->open.selected, sizeof(int32_t), hipMemcpyDeviceToHost),
+                "selected rows");
+    return 0;
+}
 
 int qs_batch_set_sum_in_order(qs_batch *b, int always) {
     if (!b || always < 0 || always > 1) {

@@ -46,6 +46,7 @@ struct OpenCtl {
 struct OpenScratch {
     int32_t *queue;                  // a count (zeroed by the streaming kernel), then the rows
                                      // that the decision kernel left undecided
+    int32_t *selected;               // rows decided by selection so far
     uint64_t *hist;                  // [rows][QS_OPEN_BINS]  (null: no such scratch)
     OpenSum *sum;                    // [rows][parts]
     OpenPartRec *prec;               // [rows][parts]

@@ -456,6 +456,7 @@ __device__ __forceinline__ bool open_finish(const PartArgs &a, const OpenArgs &o
         ring_record(a.st.ring + (int64_t)row * a.st.ring_stride, a.st.hlen + row,
                     a.st.hhead + row, P.ring_cap, id);
         a.out[row] = id;
+        add_dev(o.s.selected, 1);
         if (a.diag) {
             qs_pick_diag d;
             memset(&d, 0, sizeof d);

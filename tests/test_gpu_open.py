@@ -1,7 +1,9 @@
 """GPU: rows without a top-k whose kept prefix may be the whole window (qs_open.h), against
 the CPU restatement (sample.c:111-179) on the same logits: ids, the kept prefixes, the
 drawn position, the softmax normaliser, generator states and histories.  All whole numbers
-(inv: a float fixed by the definition), so compared exactly."""
+(inv: a float fixed by the definition), so compared exactly.  And the batch's count of rows
+decided by selection: every whole-window row of ordinary values (flat, heavy-tailed) is one,
+so the sort serves none of them."""
 import numpy as np
 import pytest
 
@@ -9,6 +11,7 @@ pytestmark = pytest.mark.gpu
 
 # vocabularies at the part's edges (4,096 logits) and over the real range
 SIZES = [4, 60, 4092, 4096, 4100, 40960, 151936, 262144]
+ORDINARY = (0, 1, 4)                   # rows_of's rows of values that seldom repeat
 # (temperature, top_p, top_k, min_p, penalty, last_n)
 SETTINGS = [
     (1.0, 1.0, 0, 0.0, 1.0, 0), (0.7, 0.9, 0, 0.0, 1.0, 0), (1.0, 0.8, 0, 0.1, 1.2, 64),
@@ -52,7 +55,8 @@ def test_open_rows(oracle, V):
             b.config(r, 1, *SETTINGS[(first + r) // len(x)], seeds=[1000 + first + r])
         b.set_history(0, hist)
         got = [b.pick(buf.ptr, V, m, V, diag=True) for _ in range(2)]
-        paths = {}
+        selected = b.selected_rows()
+        paths, whole, ordinary = {}, 0, 0
         for r in range(m):
             s = oracle.sampler()
             cfg = SETTINGS[(first + r) // len(x)]
@@ -65,13 +69,16 @@ def test_open_rows(oracle, V):
                 assert int(ids[r]) == want, at
                 assert d.keep == od["keep"], at
                 if d.path == qa.PATH_FULL:
+                    whole += 1
+                    ordinary += (first + r) % len(x) in ORDINARY
                     assert np.float32(d.inv) == np.float32(od["inv"]) or np.isnan(od["inv"]), at
                     assert (d.keep_topp, d.n_window, d.rank) == \
                         (od["keep_topp"], od["n_window"], od["rank"]), at
                 paths[d.path] = paths.get(d.path, 0) + 1
             rng, h = b.get_state(r)
             assert rng == s.rng and (h == s.history()).all(), at
-        print(V, first, "paths", paths, flush=True)
+        print(V, first, "paths", paths, "selected", selected, "ordinary", ordinary, flush=True)
+        assert ordinary <= selected <= whole
         b.close()
         buf.free()
 
@@ -90,6 +97,8 @@ def test_open_rows_summed_in_id_order(oracle, V):
         b.set_sum_in_order(1)
         b.config(0, B, *cfg, seeds=np.arange(7, 7 + B))
         got = [b.pick(dev.ptr, V, B, V, diag=True) for _ in range(2)]
+        ordinary = sum(got[k][1][r].path == qa.PATH_FULL for k in range(2) for r in range(3))
+        assert b.selected_rows() >= ordinary, cfg
         for r in range(B):
             s = oracle.sampler()
             s.config(*cfg, seed=7 + r)
