@@ -289,6 +289,10 @@ int qs_batch_set_spin_limit(qs_batch *b, int attempts);
  * equals the reference's bit for bit); 0, the default, only where needed. */
 int qs_batch_set_sum_in_order(qs_batch *b, int always);
 
+/* A test hook: the next n launches of the whole-window decision (process-wide) fail, after the
+ * pick's other kernels were enqueued: the pick returns QS_EDEVICE.  0, or QS_EINVAL for n < 0. */
+int qs_debug_fail_open_launches(int n);
+
 /* QS_PATH_FULL rows since the batch was made that were decided by selecting the two positions
  * of their whole window, not by sorting it (a test hook; waits for the batch's stream). */
 int qs_batch_selected_rows(qs_batch *b, int *n);

@@ -58,6 +58,7 @@ PROTOS = [
     ("qs_pick_noalloc", _i, [_vp, _i64, _i, _i, _vp, _vp, _vp, _i, _vp, _vp, _vp, _vp]),
     ("qs_batch_set_spin_limit", _i, [_vp, _i]),
     ("qs_batch_set_sum_in_order", _i, [_vp, _i]),
+    ("qs_debug_fail_open_launches", _i, [_i]),
     ("qs_batch_selected_rows", _i, [_vp, C.POINTER(C.c_int)]),
     ("qs_last_error", C.c_char_p, []),
     ("qs_device_alloc", _vp, [_sz]),

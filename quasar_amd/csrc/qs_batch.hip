@@ -627,8 +627,8 @@ struct qs_batch {
     OpenScratch open{};                    // rows without a top-k (allocated when one is
                                            // configured)
     void *d_open = nullptr;                // its one allocation
-    bool open_dirty = false;               // a launch failed between its two kernels: its
-                                           // counters are cleared before the next pick
+    bool open_dirty = false;               // a launch failed between its kernels: cleared
+                                           // before the next pick that uses it
     // Pinned host memory the kernels write: the error flag, then a pick's ids (max_rows).
     // The host reads both after its one wait on the stream, with no copy back: a blocking
     // 4-byte copy costs about 13 us, and a pick of 32 rows needed two.
@@ -1014,11 +1014,11 @@ static int pick_range(qs_batch *b, int row0, const float *d_logits, int64_t row_
             HIP_TRY(hipMemset(b->open.ctl, 0, sizeof(OpenCtl) * R), "open rows");
             HIP_TRY(hipStreamSynchronize(nullptr), "open rows");
         }
-        b->open_dirty = open;
+        if (open) b->open_dirty = true;
         const int rc = qs_part_launch(d_logits, row_stride, n_rows, n_vocab, st0, b->sc, d_out,
                                       d_diag, b->part_resident, b->stream, b->mid, !any_sample,
                                       open ? &b->open : nullptr);
-        if (rc == 0) b->open_dirty = false;
+        if (open && rc == 0) b->open_dirty = false;
         return rc;
     }
     Geometry g;

@@ -37,6 +37,7 @@ void qs_default_param(qs_row_param *out, uint64_t *rng_out);
 /* Fault injection for tests: nonzero while injected device failures remain (each call
  * consumes one); see qs_debug_fail_picks. */
 int qs_debug_take_failure(void);
+int qs_debug_take_open_failure(void);     /* the same for qs_debug_fail_open_launches */
 
 /* sample.h's pick of one row in one round trip: the host row copied to d_logits on the
  * batch's stream, then qs_batch_pick_ids: the kernels write the id (and the batch's error

@@ -49,6 +49,23 @@ int qs_debug_fail_picks(int n) {
     return 0;
 }
 
+static int qs_open_fail_left;   /* injected failures of k_open's launch */
+
+int qs_debug_fail_open_launches(int n) {
+    if (n < 0) { qs_set_error("qs_debug_fail_open_launches: n %d", n); return QS_EINVAL; }
+    __atomic_store_n(&qs_open_fail_left, n, __ATOMIC_RELAXED);
+    return 0;
+}
+
+int qs_debug_take_open_failure(void) {
+    int left = __atomic_load_n(&qs_open_fail_left, __ATOMIC_RELAXED);
+    while (left > 0)
+        if (__atomic_compare_exchange_n(&qs_open_fail_left, &left, left - 1, 0,
+                                        __ATOMIC_RELAXED, __ATOMIC_RELAXED))
+            return 1;
+    return 0;
+}
+
 int qs_debug_take_failure(void) {
     int v = __atomic_load_n(&qs_fail_left, __ATOMIC_RELAXED);
     while (v > 0) {

@@ -1472,6 +1472,7 @@ int qs_part_launch(const float *logits, int64_t row_stride, int n_rows, int n_vo
             hipLaunchKernelGGL(k_open_sum, dim3(np), dim3(ND), 0, stream, a, oa);
             e = hipGetLastError();
         }
+        if (open && qs_debug_take_open_failure()) e = hipErrorLaunchFailure;
         if (e == hipSuccess && open) {
             hipLaunchKernelGGL(unal ? k_open<true> : k_open<false>, dim3(np), dim3(ND), 0, stream,
                                a, oa);

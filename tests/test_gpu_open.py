@@ -139,3 +139,32 @@ def test_certified_rows_without_a_top_k_pay_empty_launches_only(B):
     assert us[1 << 20] <= 1.25 * us[0]
     b.close()
     dev.free()
+
+
+def test_scratch_is_cleared_after_a_failed_launch():
+    """The whole-window launch failing after the first pass has filled its histograms, then a
+    pick that does not use them, then whole-window rows of other logits: decided by selection,
+    as no pick on the failed one's histograms would be."""
+    import quasar_amd as qa
+    V, B = 40960, 8
+    r = np.random.default_rng(8)
+    wide = qa.DeviceBuffer.from_array((r.normal(0, 1, (B, V)) * 6).astype(np.float32))
+    flat = qa.DeviceBuffer.from_array(r.normal(0, 1, (B, V)).astype(np.float32))
+    b = qa.Batch(B, V, 8)
+    open_rows = dict(temperature=1.0, top_p=0.9, top_k=0, seeds=np.arange(1, B + 1))
+    b.config(0, B, **open_rows)
+    want = b.pick(flat.ptr, V, B, V)
+    assert b.selected_rows() == B
+    b.config(0, B, temperature=3.0, top_p=0.9, top_k=0, seeds=np.arange(1, B + 1))
+    qa.check(qa.load().qs_debug_fail_open_launches(1), "qs_debug_fail_open_launches")
+    with pytest.raises(qa.QsError) as e:
+        b.pick(wide.ptr, V, B, V)
+    assert e.value.rc == qa._native.QS_EDEVICE
+    b.config(0, B, temperature=1.0, top_k=5, seeds=np.arange(1, B + 1))
+    b.pick(flat.ptr, V, B, V)
+    b.config(0, B, **open_rows)
+    assert (b.pick(flat.ptr, V, B, V) == want).all()
+    assert b.selected_rows() == 2 * B
+    b.close()
+    wide.free()
+    flat.free()
