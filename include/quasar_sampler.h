@@ -172,8 +172,10 @@ int qs_batch_pick_ids(qs_batch *b, const float *d_logits, int64_t row_stride, in
 
 /* Which kernels qs_batch_pick uses.  AUTO (the default) takes the row kernel for batches
  * of at least a quarter of a row per CU whose sampling rows have a top-k of at most 256 (or top-k
- * off), the streaming kernels for smaller batches, larger top-k and rows at any other
- * alignment, and the split-row kernels for vocabularies neither supports.  ROW: one kernel, one workgroup per row,
+ * off), the streaming kernels for smaller batches, larger top-k and sampling rows of 25,600
+ * logits or more at any other alignment (35,840 and 195 times the top-k past 64; 10,240 for up
+ * to 64 rows with one whose top-k is off), and the split-row kernels for the rest.  ROW: one
+ * kernel, one workgroup per row,
  * every logit read once and the row decided from LDS (16-byte aligned rows, a vocabulary
  * and a row stride that are multiples of 4, vocabulary up to 262,144).  STREAM: two
  * kernels, every logit read once by workgroups that each take a part of a row, then one

@@ -771,25 +771,52 @@ static bool rows_ok(const qs_batch *b, int row0, int n_rows) {
     return true;
 }
 
+// Whether AUTO streams a pick of rows that are not 16-byte aligned.  A part keeps about twice
+// its share of a row's candidates, so a row of few parts often falls short of them (or
+// overflows a part's lists) and decides over its whole window; the split-row kernels, which
+// gather from slices of the whole row, do not.  Microseconds a pick, split / streaming, means
+// over 4 to 10 inputs:
+//   every row greedy: 1 row 6.7 / 10.1, 100 rows of 100,003 16.9 / 22.6, 1024 rows 103 / 118;
+//   top-k up to 64 or off: 32 rows of 12,289 logits 20 / 67 to 115, of 28,001 38 / 18, of
+//     100,277 44 / 23; 512 rows of 4,099 24 / 88, of 28,001 331 / 38, of 100,277 2117 / 70;
+//   top-k 128: 32 rows of 24,001 37 / 93, of 36,001 40 / 25; 512 of 36,001 80 / 119 (128: 173 /
+//     25); top-k 200: 32 of 32,001 82 / 270, of 40,963 82 / 31; 400: 32 of 60,001 835 / 431;
+//     512: 32 of 60,001 441 / 930, of 100,277 674 / 171;
+//   a row without a top-k, up to QS_OPEN_ROWS rows (such a row has qs_open.h): top-p 0.9, 32
+//     rows of 12,289 315 / 31, of 8,191 146 / 36, but min-p 0.05, which needs no window, 19 / 19
+//     and 18 / 29.
+//   min-p on 2,048 rows of 1,001 logits: 44 us / 24 ms.
+static bool unaligned_streams(const qs_batch *b, int row0, int n_rows, int n_vocab, int kmax,
+                              bool any_sample) {
+    if (!any_sample) return false;
+    constexpr int part = QS_PART_LEN;
+    if (kmax > 64) return n_vocab >= 7 * part / 2 && n_vocab >= 195 * kmax;
+    if (n_vocab >= 5 * part / 2) return true;
+    if (n_vocab < part || n_rows > QS_OPEN_ROWS || !b->d_open) return false;
+    for (int r = row0; r < row0 + n_rows; ++r)
+        if (qs_open_row(b->h_prm[r], n_vocab)) return true;
+    return false;
+}
+
 // The kernels a pick with these arguments takes: the batch's mode, or for AUTO the row
 // kernel when the batch has a row for at least a quarter of the CUs and every sampling row
 // aims at most QS_ROW_AUTO_KSEL candidates (its per-wavefront candidate lists hold a few
 // hundred entries; a row that overflows them takes the full-window path), the streaming
-// kernels otherwise (rows at any alignment; the split-row kernels took 44 us for 48 rows of
-// 100,003 logits where they take 21), the split-row kernels for vocabularies below 4 or past
-// their parts.  `kmax` is the largest
+// kernels otherwise for aligned rows and, where unaligned_streams says so, for others, the
+// split-row kernels for the rest.  `kmax` is the largest
 // candidate target among the sampling rows (1 when every row is greedy).  The quarter: on
 // MI355X (256 CUs) at 151,936 logits a row, a pick of the row kernel takes about 23 us
 // from 8 to 64 rows (one workgroup per row, each row's latency), the streaming pair 17 us at
 // 8 rows rising to 22 at 48 and 28 at 64.
 static int auto_mode(const qs_batch *b, const float *d_logits, int64_t row_stride, int n_rows,
-                     int n_vocab, int kmax) {
+                     int n_vocab, int kmax, bool any_sample, int row0) {
     if (b->mode != QS_MODE_AUTO) return b->mode;
     if (4 * (int64_t)n_rows >= b->n_cu && kmax <= QS_ROW_AUTO_KSEL &&
         qs_row_supported(n_rows, n_vocab, row_stride, d_logits))
         return QS_MODE_ROW;
     return qs_part_supported(n_rows, n_vocab, row_stride, d_logits) ||
-                   qs_part_takes(n_rows, n_vocab, d_logits)
+                   (qs_part_takes(n_rows, n_vocab, d_logits) &&
+                    unaligned_streams(b, row0, n_rows, n_vocab, kmax, any_sample))
                ? QS_MODE_STREAM
                : QS_MODE_SPLIT;
 }
@@ -963,7 +990,7 @@ int qs_batch_resolve_mode(qs_batch *b, const float *d_logits, int64_t row_stride
     int kmax = 1;
     bool any_sample = false;
     if (const int rc = batch_kmax(b, n_rows, &kmax, &any_sample)) return rc;
-    return auto_mode(b, d_logits, row_stride, n_rows, n_vocab, kmax);
+    return auto_mode(b, d_logits, row_stride, n_rows, n_vocab, kmax, any_sample, 0);
 }
 
 // The pick of the batch's rows [row0, row0 + n_rows) from logits rows 0 .. n_rows - 1: the
@@ -985,7 +1012,8 @@ static int pick_range(qs_batch *b, int row0, const float *d_logits, int64_t row_
     const int rs = b->max_last_n > 0 ? b->max_last_n : 1;
     RowState st0{b->d_prm + row0, b->d_rng + row0, b->d_ring + (int64_t)row0 * rs,
                  b->d_hlen + row0, b->d_hhead + row0, rs};
-    const int mode = auto_mode(b, d_logits, row_stride, n_rows, n_vocab, kmax);
+    const int mode =
+        auto_mode(b, d_logits, row_stride, n_rows, n_vocab, kmax, any_sample, row0);
     if (mode == QS_MODE_ROW) {
         if (!qs_row_supported(n_rows, n_vocab, row_stride, d_logits)) {
             qs_set_error("qs_batch_pick: the row kernel does not support this pick");

@@ -13,6 +13,7 @@
 // Parts per row the streaming kernel supports (lanes of its row decision), wavefronts of
 // its workgroups (one candidate list each) and candidates per part.
 #define QS_PART_MAX_PARTS 64
+#define QS_PART_LEN 10240
 #define QS_PART_WAVES 8
 #define QS_PART_CANDS 256
 
@@ -60,8 +61,8 @@ bool qs_open_row(const qs_row_param &p, int n_vocab);
 // Whether the streaming kernel handles this pick (16-byte aligned rows, vocabulary and row
 // stride multiples of 4, at most QS_PART_MAX_PARTS parts).
 int qs_part_supported(int n_rows, int n_vocab, int64_t row_stride, const void *logits);
-// Whether it takes the pick with rows at any alignment (float-aligned logits, a vocabulary of
-// at least 4): what AUTO asks; the callers that demand aligned rows keep qs_part_supported.
+// Whether it can take the pick with rows at any alignment (float-aligned logits, a vocabulary
+// of at least 4): AUTO's; the callers that demand aligned rows keep qs_part_supported.
 int qs_part_takes(int n_rows, int n_vocab, const void *logits);
 // Parts per row at this vocabulary (the per-part scratch needs rows * parts entries).
 int qs_part_parts(int n_vocab);

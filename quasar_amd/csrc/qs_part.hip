@@ -52,6 +52,7 @@ constexpr int NWV = NT / 64;         // its wavefronts
 constexpr int UP = 5;                // float4 per thread per part
 constexpr int STAGES = 1;            // parts whose loads are in flight during one part
 constexpr int PART_MAX = NT * UP * 4;    // longest part (elements)
+static_assert(PART_MAX == QS_PART_LEN, "the length the host knows");
 constexpr int WCAP = 32;             // candidates per wavefront list
 constexpr int PCAP = NWV * WCAP;     // candidates per part
 static_assert(NWV == QS_PART_WAVES && PCAP == QS_PART_CANDS, "scratch layout");
@@ -423,6 +424,7 @@ __device__ __forceinline__ void part_step(float4 (&buf)[UP], const StreamArgs &a
     }
     const uint32_t wmn = wave_min_u(r.mn == INFINITY ? 0xFFFFFFFFu : f2key(r.mn));
     const int wnan = __ballot(r.nan != 0) ? wave_sum_i(r.nan) : 0;
+    static_assert(!(GF && UNAL), "an all-greedy pick of aligned rows");
     const bool gfuse = GF && greedy;               // (GF: every row of the pick is greedy)
     if (gfuse) {
         // sample.c:130-132 over this wavefront's share: the largest penalised logit, the
@@ -436,10 +438,8 @@ __device__ __forceinline__ void part_step(float4 (&buf)[UP], const StreamArgs &a
 #pragma unroll
             for (int k = 0; k < 4; ++k) {
                 const uint32_t wk = f2key(w[k] == 0.0f ? 0.0f : w[k]);
-                const uint64_t gk =
-                    ((uint64_t)wk << 32) | (uint32_t)~(uint32_t)(4 * c + k - l.sh);
-                const bool in = UNAL ? is_logit(a, l, 4 * c + k) : c < l.c_hi;
-                if (in && w[k] == w[k] && gk > g) g = gk;
+                const uint64_t gk = ((uint64_t)wk << 32) | (uint32_t)~(uint32_t)(4 * c + k);
+                if (c < l.c_hi && w[k] == w[k] && gk > g) g = gk;
             }
         }
         g = wave_reduce(g, [](uint64_t x, uint64_t y) { return x > y ? x : y; });
@@ -1439,13 +1439,11 @@ int qs_part_launch(const float *logits, int64_t row_stride, int n_rows, int n_vo
     if (a.xcd_map) grid = grid / 8 * 8;
     if (grid > total) grid = a.xcd_map ? (total + 7) / 8 * 8 : total;
     if (grid < 1) grid = 1;
-    // every row greedy, with the scratch for it: each row decided by its last part
-    const bool gf = all_greedy && sc.gbest != nullptr;
-    const dim3 parts_grid((unsigned)grid);
-    hipLaunchKernelGGL(gf ? (unal ? k_part<true, true> : k_part<true, false>)
-                          : (unal ? k_part<false, true> : k_part<false, false>),
-                       parts_grid, dim3(NT), 0, stream, sa, sa.logits, sa.prm, sa.ring, sa.hlen,
-                       sa.hhead, sa.rec, sa.cand);
+    // every row greedy and aligned, with the scratch for it: each decided by its last part
+    const bool gf = all_greedy && sc.gbest != nullptr && !unal;
+    auto *kp = gf ? k_part<true, false> : unal ? k_part<false, true> : k_part<false, false>;
+    hipLaunchKernelGGL(kp, dim3((unsigned)grid), dim3(NT), 0, stream, sa, sa.logits, sa.prm, sa.ring,
+                       sa.hlen, sa.hhead, sa.rec, sa.cand);
     hipError_t e = hipGetLastError();
     if (e == hipSuccess && mid) e = hipEventRecord(mid, stream);
     if (e == hipSuccess && !gf) {
