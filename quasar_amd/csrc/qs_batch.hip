@@ -1239,11 +1239,7 @@ int qs_batch_head_logits(qs_batch *b, const void *d_hidden, const void *d_weight
     if (const int rc = head_check(b, d_hidden, d_weight, n_embd, n_rows, n_vocab, d_logits,
                                   false))
         return rc;
-    // Up to one 128-column tile a CU there is nothing to balance, and the tile kernels, with
-    // half the columns a stage, take less time (V = 32,000: 1 row x 512 6.6 us against 7.4, 40
-    // rows x 4096 43 against 45, 256 x 4096 91 against 100); past it qs_logits.hip's runs do
-    // (200 rows x 1024 x 50,000: 36 us against 43).
-    if ((n_vocab + QS_HEAD_TILE - 1) / QS_HEAD_TILE > b->n_cu &&
+    if (qs_logits_pays(n_embd, n_rows, n_vocab, b->n_cu) &&
         qs_logits_fits(n_embd, n_rows, n_vocab, b->n_cu))
         return qs_logits_launch(d_hidden, d_weight, n_embd, n_rows, n_vocab, d_logits, b->n_cu,
                                 b->stream);

@@ -153,6 +153,8 @@ size_t qs_head_packed_elems(int n_embd, int n_vocab);
 // output-layer kernel reads (qs_head_packed_elems elements at d_packed).
 int qs_head_pack_launch(const void *d_weight, int n_embd, int n_vocab, void *d_packed,
                         hipStream_t stream);
+// Whether qs_logits_launch takes less time than the tile kernels of qs_head.hip.
+bool qs_logits_pays(int n_embd, int n_rows, int n_vocab, int n_cu);
 // Whether qs_logits_launch can address this layer: a workgroup's run of W and the hidden rows
 // each lie within one buffer (under 4 GiB).  No device of 288 GB holds a layer that does not.
 bool qs_logits_fits(int n_embd, int n_rows, int n_vocab, int n_cu);

@@ -279,8 +279,32 @@ LIN_KERNEL(256)
 // (128 rows x 512 x 151,936, 156 + 78 MB: 41.5 against 46.8 us; 256 x 1024 x 80,000, 164 + 82
 // MB: 58 against 64; at 205 + 3 MB the two are even).
 constexpr uint64_t NT_BYTES = 256ull << 20;
+uint64_t layer_bytes(int n_embd, int n_rows, int n_vocab) {
+    return (2ull * (uint64_t)n_embd + 4ull * (uint64_t)n_rows) * (uint64_t)n_vocab;
+}
 
 }  // namespace
+
+// Microseconds, the tile kernels / this file's, W from HBM (matrices in turn past the last-level
+// cache) unless said otherwise:
+//   * up to one 128-column tile a CU there is nothing to balance (V = 32,000: 1 row x 512 6.6 /
+//     7.4, 40 rows x 4096 43 / 45, 256 x 4096 91 / 100);
+//   * a short run is all ramp: E = 64, 1 row 4.0 / 4.8 at V = 32,772, 7.0 / 8.0 at 128,256; 64
+//     rows x 256 11.5 / 12.3 at 64,000, 23.3 / 24.8 at 151,936.  128 rows x 256 13.7 / 10.9 at
+//     32,772, 33.1 / 31.7 at 151,936; 64 rows x 512 15.2 / 12.5 and 38.2 / 36.8;
+//   * up to 64 rows that do not pass the last-level cache, the tiles (two a CU at once) lose
+//     only in a round that is not full: 1 row x 512 at 1,002 tiles of 1,024 places (V = 128,256)
+//     24.9 / 27.1, in the cache 21.4 / 22.1, at 500 of 512 (64,000) 14.4 / 14.5 and 12.2 / 13.4;
+//     at 782 of 1,024 (100,000) 22.6 / 20.9 and 19.1 / 18.2, at 257 of 512 11.5 / 10.4.
+// Past it: 1 row x 2048 x 128,256 89 / 81, 64 rows x 2048 x 100,000 100 / 78 (128,256 x 1536 is
+// the exception: 68 / 77 at 1 row, 111 / 107 at 128).
+bool qs_logits_pays(int n_embd, int n_rows, int n_vocab, int n_cu) {
+    const int tiles = (n_vocab + LT - 1) / LT, places = 2 * n_cu;
+    if (tiles <= n_cu || n_embd < 256) return false;
+    if (n_rows > 64 || layer_bytes(n_embd, n_rows, n_vocab) > NT_BYTES) return true;
+    const int rounds = (tiles + places - 1) / places;
+    return n_embd >= 512 && 20 * (int64_t)tiles < 19 * (int64_t)rounds * places;
+}
 
 bool qs_logits_fits(int n_embd, int n_rows, int n_vocab, int n_cu) {
     // (a run of ceil(blocks / n_cu) blocks of 32 columns touches at most this many tiles)
@@ -302,7 +326,7 @@ int qs_logits_launch(const void *d_hidden, const void *d_weight, int n_embd, int
     a.logits = d_logits;
     const unsigned grid = (unsigned)n_cu;             // (n_vocab > 128 n_cu)
     // the smallest row capacity that holds the batch (the H stages take less of the LDS)
-    const bool nt = (2ull * (uint64_t)n_embd + 4ull * (uint64_t)n_rows) * (uint64_t)n_vocab > NT_BYTES;
+    const bool nt = layer_bytes(n_embd, n_rows, n_vocab) > NT_BYTES;
     auto *k = n_rows <= 32    ? (nt ? k_logits32_nt : k_logits32)
               : n_rows <= 64  ? (nt ? k_logits64_nt : k_logits64)
               : n_rows <= 128 ? (nt ? k_logits128_nt : k_logits128)

@@ -1,7 +1,7 @@
-"""GPU: the output layer alone where every CU takes a run of columns (qs_logits.hip:
-vocabularies past one 128-column tile a CU), against a float64 product within the bound of
-any fp32 summation order of exact bf16 products, E 2^-24 sum |h w|, and bit for bit against
-the fused kernels' logits, which add in the same order."""
+"""GPU: the output layer alone, where every CU takes a run of columns (qs_logits.hip: past one
+128-column tile a CU, from 256 embedding elements on) and in its tiles, against a float64
+product within the bound of any fp32 summation order of exact bf16 products, E 2^-24 sum |h w|,
+and bit for bit against the fused kernels' logits, which add in the same order."""
 import numpy as np
 import pytest
 import torch
@@ -12,7 +12,11 @@ pytestmark = pytest.mark.gpu
 @pytest.mark.parametrize("rows,E,V", [
     (1, 64, 32772), (31, 64, 33000), (32, 128, 40960), (33, 192, 32800), (64, 512, 65536),
     (65, 64, 151936), (100, 320, 81920), (128, 128, 90004), (129, 64, 32772), (200, 192, 50000),
-    (255, 256, 98304), (256, 64, 262144), (256, 512, 81924), (16, 2048, 60000)])
+    (255, 256, 98304), (256, 64, 262144), (256, 512, 81924), (16, 2048, 60000),
+    # the runs at the edges of their row shapes
+    (1, 512, 32772), (31, 512, 33000), (32, 576, 40960), (33, 512, 32800), (64, 512, 90004),
+    (65, 256, 151936), (100, 320, 40960), (128, 256, 90004), (129, 256, 32772), (200, 256, 50000),
+    (256, 256, 262144)])
 def test_logits_of_column_runs(rows, E, V):
     import quasar_amd as qa
     g = torch.Generator(device="cuda")
