@@ -1074,20 +1074,9 @@ __global__ void __launch_bounds__(ND) k_decide(PartArgs a, open::OpenArgs o) {
     if (tid < QS_EXPF_TAB_N) dl.dl.tab[tid] = c_tab_part[tid];
     RowHist hist{0ull, 0, 0};
     if (tid < 64 && !greedy) hist = row_hist(st, row);
-    // a row the certified decision does not cover: queued for k_open, or decided here
     if (OPEN && tid == 0) o.s.ctl[row].reason = 0;
-    auto undecided = [&](const CertTotals &t, int reason) __attribute__((always_inline)) {
-        if constexpr (OPEN) {
-            if (open::open_row(P, a.vocab) && isfinite(t.msc)) {
-                if (tid == 0) {
-                    o.s.ctl[row].reason = reason;
-                    o.s.queue[1 + add_dev(o.s.queue, 1)] = row;
-                }
-                return;
-            }
-        }
-        exact_row<UNAL>(a, row, P, t, dl, hist, reason);
-    };
+    CertTotals t;
+    int status;
     if (NL <= 128) {
         // rows of up to 16 parts: greedy rows by wavefront 0 alone, sampling rows by the
         // workgroup (decide_par); the whole workgroup then takes the block decision, a
@@ -1115,200 +1104,180 @@ __global__ void __launch_bounds__(ND) k_decide(PartArgs a, open::OpenArgs o) {
             if (tid == 0) record_greedy(row, P, bv, bi, dl.ct.maxl, x[0], st, a.out, a.diag);
             return;
         }
-        CertTotals t = dl.ct;
-        int status = s0;
-        if (s0 == DS_BLOCK) {
-            status = cert_row_block<ND>(row, P, t, dl.keys, dl.ids, dl.srt, dl.dl, st, a.out,
-                                        a.diag, hist);
-            if (status == 0) return;
-        }
-        if (WIDE && widen_pays(status, P, t) && widen<UNAL>(a, row, P, dl)) {
-            t = dl.ct;
-            if (row_ksel(P) <= 64 && t.total <= WAVE_CAND) {
-                if (wv == 0) {
-                    const int s1 = cert_row_wave(row, P, t, dl.keys, dl.ids, dl.srt, dl.dl.tab,
-                                                 st, a.out, a.diag, hist);
-                    if (lane == 0) dl.dl.sh[7] = s1;
-                }
-                __syncthreads();
-                status = dl.dl.sh[7];
-                __syncthreads();
-            } else {
-                status = cert_row_block<ND>(row, P, t, dl.keys, dl.ids, dl.srt, dl.dl, st, a.out,
-                                            a.diag, hist);
-            }
-            if (status == 0) return;
-        }
-        undecided(t, status);
-        return;
-    }
-    // records and lists tid and ND + tid (number L: wavefront L mod 8 of part L / 8, its
-    // candidates at (l0*8 + L)*WCAP), with the first SPEC candidates: one round trip
-    constexpr int SPEC = 8;
-    WaveRec rec[2];
-    uint4 spec[2][SPEC / 2];
-#pragma unroll
-    for (int h = 0; h < 2; ++h) {
-        const int L = h * ND + tid;
-        if (L < NL) {
-            rec[h] = sc.wrec[(int64_t)l0 * NWV + L];
-            const uint4 *src = (const uint4 *)(sc.pcand + ((int64_t)l0 * NWV + L) * WCAP);
-#pragma unroll
-            for (int i = 0; i < SPEC / 2; ++i) spec[h][i] = src[i];
-        } else {
-            rec[h].sum = 0.0;
-            rec[h].term = 0.0f;
-            rec[h].mink = 0xFFFFFFFFu;
-            rec[h].nan = 0;
-            rec[h].maxk = 0u;
-            rec[h].rej = 0u;
-            rec[h].cnt = 0;
-        }
-    }
-    // each part's totals from its NWV wavefront records (consecutive lanes, a fixed order)
-#pragma unroll
-    for (int h = 0; h < 2; ++h) {
-        double ps = rec[h].sum;
-        float pt = rec[h].term;
-        uint32_t pmn = rec[h].mink;
-        int pn = rec[h].nan;
-#pragma unroll
-        for (int o = 1; o < NWV; o <<= 1) {
-            ps += __shfl_xor(ps, o, 64);
-            pt += __shfl_xor(pt, o, 64);
-            pmn = min(pmn, (uint32_t)__shfl_xor((int)pmn, o, 64));
-            pn += __shfl_xor(pn, o, 64);
-        }
-        const int L = h * ND + tid;
-        if ((tid & (NWV - 1)) == 0 && L < NL) {
-            const int j = L / NWV;
-            dl.pmaxk[j] = rec[h].maxk;
-            dl.prej[j] = rec[h].rej;
-            dl.psum[j] = ps;
-            dl.pterm[j] = pt;
-            dl.pmin[j] = pmn;
-            dl.pnan[j] = pn;
-        }
-    }
-    __syncthreads();
-    if (tid < 64) {
-        const bool have = lane < NP;
-        const uint32_t mk = have ? dl.pmaxk[lane] : 0u;
-        const uint32_t rmx = wave_max_u(mk);
-        const float maxl = key2f(rmx > KEY_NEG_INF ? rmx : KEY_NEG_INF);
-        const float inv_t = P.inv_t;
-        const float msc = maxl * inv_t, thr = msc - 30.0f;
-        CertPart cp{0.0, 0.0};
-        const float maxw = have ? key2f(mk > KEY_NEG_INF ? mk : KEY_NEG_INF) : -INFINITY;
-        if (!greedy && have) cp = cert_part(maxw, dl.psum[lane], dl.pterm[lane], inv_t, msc, thr);
-        const double lo = wave_sum_d(cp.lo), hi = wave_sum_d(cp.hi);
-        // window size: exact when every part lies wholly in or wholly out of it
-        const int plen = have ? part_count<UNAL>(a, row, lane) : 0;
-        const uint32_t pmn = have ? dl.pmin[lane] : 0xFFFFFFFFu;
-        const bool out_j = !(maxw * inv_t >= thr);
-        const bool in_j = have && pmn != 0xFFFFFFFFu && key2f(pmn) * inv_t >= thr;
-        const bool known = __ballot(have && !out_j && !in_j) == 0ull;
-        const int nin = wave_sum_i(have && !out_j && in_j ? plen - dl.pnan[lane] : 0);
-        const uint32_t rj = wave_max_u(have ? dl.prej[lane] : 0u);
-        if (lane == 0) {
-            CertTotals t;
-            t.maxl = maxl;
-            t.msc = msc;
-            double S_lo = 1.0, S_hi = 1.0;
-            if (!greedy) cert_interval(lo, hi, msc, thr, a.vocab, S_lo, S_hi);
-            t.S_lo = S_lo;
-            t.S_hi = S_hi;
-            t.v_lo = (float)(1.0 / S_hi);
-            t.v_hi = (float)(1.0 / S_lo);
-            t.nwin = known ? nin : -1;
-            t.cflag = 0;
-            t.rej = rj;
-            t.total = 0;
-            dl.ct = t;
-        }
-    }
-    const int cnt0 = rec[0].cnt, cnt1 = rec[1].cnt;
-    const int c0 = min(cnt0, WCAP), c1 = min(cnt1, WCAP);
-    const int ovf = __ballot(cnt0 > WCAP || cnt1 > WCAP) != 0ull;
-    // f(entry, list h, position) over the entries of lists tid and ND + tid
-    auto each_entry = [&](auto &&f) {
+        t = dl.ct;
+        status = s0;
+    } else {
+        // records and lists tid and ND + tid (number L: wavefront L mod 8 of part L / 8, its
+        // candidates at (l0*8 + L)*WCAP), with the first SPEC candidates: one round trip
+        constexpr int SPEC = 8;
+        WaveRec rec[2];
+        uint4 spec[2][SPEC / 2];
 #pragma unroll
         for (int h = 0; h < 2; ++h) {
-            const int n = h ? c1 : c0;
+            const int L = h * ND + tid;
+            if (L < NL) {
+                rec[h] = sc.wrec[(int64_t)l0 * NWV + L];
+                const uint4 *src = (const uint4 *)(sc.pcand + ((int64_t)l0 * NWV + L) * WCAP);
 #pragma unroll
-            for (int i = 0; i < SPEC; ++i)
-                if (i < n) {
-                    const uint4 q = spec[h][i >> 1];
-                    f((i & 1) ? make_uint2(q.z, q.w) : make_uint2(q.x, q.y), h, i);
-                }
-            const uint2 *src = sc.pcand + ((int64_t)l0 * NWV + h * ND + tid) * WCAP;
-            for (int i = SPEC; i < n; ++i) f(src[i], h, i);
+                for (int i = 0; i < SPEC / 2; ++i) spec[h][i] = src[i];
+            } else {
+                rec[h].sum = 0.0;
+                rec[h].term = 0.0f;
+                rec[h].mink = 0xFFFFFFFFu;
+                rec[h].nan = 0;
+                rec[h].maxk = 0u;
+                rec[h].rej = 0u;
+                rec[h].cnt = 0;
+            }
         }
-    };
-    if (greedy) {
-        // the first largest penalised logit (sample.c:130-132): every part's maxima are
-        // among its candidates unless a list overflowed; then the row is scanned
-        float bv = -INFINITY;
-        int bi = -1;
-        each_entry([&](uint2 e, int, int) { best_combine(bv, bi, key2f(e.x), (int)e.y); });
+        // each part's totals from its NWV wavefront records (consecutive lanes, a fixed order)
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+            double ps = rec[h].sum;
+            float pt = rec[h].term;
+            uint32_t pmn = rec[h].mink;
+            int pn = rec[h].nan;
+#pragma unroll
+            for (int o = 1; o < NWV; o <<= 1) {
+                ps += __shfl_xor(ps, o, 64);
+                pt += __shfl_xor(pt, o, 64);
+                pmn = min(pmn, (uint32_t)__shfl_xor((int)pmn, o, 64));
+                pn += __shfl_xor(pn, o, 64);
+            }
+            const int L = h * ND + tid;
+            if ((tid & (NWV - 1)) == 0 && L < NL) {
+                const int j = L / NWV;
+                dl.pmaxk[j] = rec[h].maxk;
+                dl.prej[j] = rec[h].rej;
+                dl.psum[j] = ps;
+                dl.pterm[j] = pt;
+                dl.pmin[j] = pmn;
+                dl.pnan[j] = pn;
+            }
+        }
+        __syncthreads();
+        if (tid < 64) {
+            const bool have = lane < NP;
+            const uint32_t mk = have ? dl.pmaxk[lane] : 0u;
+            const uint32_t rmx = wave_max_u(mk);
+            const float maxl = key2f(rmx > KEY_NEG_INF ? rmx : KEY_NEG_INF);
+            const float inv_t = P.inv_t;
+            const float msc = maxl * inv_t, thr = msc - 30.0f;
+            CertPart cp{0.0, 0.0};
+            const float maxw = have ? key2f(mk > KEY_NEG_INF ? mk : KEY_NEG_INF) : -INFINITY;
+            if (!greedy && have) cp = cert_part(maxw, dl.psum[lane], dl.pterm[lane], inv_t, msc, thr);
+            const double lo = wave_sum_d(cp.lo), hi = wave_sum_d(cp.hi);
+            // window size: exact when every part lies wholly in or wholly out of it
+            const int plen = have ? part_count<UNAL>(a, row, lane) : 0;
+            const uint32_t pmn = have ? dl.pmin[lane] : 0xFFFFFFFFu;
+            const bool out_j = !(maxw * inv_t >= thr);
+            const bool in_j = have && pmn != 0xFFFFFFFFu && key2f(pmn) * inv_t >= thr;
+            const bool known = __ballot(have && !out_j && !in_j) == 0ull;
+            const int nin = wave_sum_i(have && !out_j && in_j ? plen - dl.pnan[lane] : 0);
+            const uint32_t rj = wave_max_u(have ? dl.prej[lane] : 0u);
+            if (lane == 0) {
+                CertTotals t;
+                t.maxl = maxl;
+                t.msc = msc;
+                double S_lo = 1.0, S_hi = 1.0;
+                if (!greedy) cert_interval(lo, hi, msc, thr, a.vocab, S_lo, S_hi);
+                t.S_lo = S_lo;
+                t.S_hi = S_hi;
+                t.v_lo = (float)(1.0 / S_hi);
+                t.v_hi = (float)(1.0 / S_lo);
+                t.nwin = known ? nin : -1;
+                t.cflag = 0;
+                t.rej = rj;
+                t.total = 0;
+                dl.ct = t;
+            }
+        }
+        const int cnt0 = rec[0].cnt, cnt1 = rec[1].cnt;
+        const int c0 = min(cnt0, WCAP), c1 = min(cnt1, WCAP);
+        const int ovf = __ballot(cnt0 > WCAP || cnt1 > WCAP) != 0ull;
+        // f(entry, list h, position) over the entries of lists tid and ND + tid
+        auto each_entry = [&](auto &&f) {
+#pragma unroll
+            for (int h = 0; h < 2; ++h) {
+                const int n = h ? c1 : c0;
+#pragma unroll
+                for (int i = 0; i < SPEC; ++i)
+                    if (i < n) {
+                        const uint4 q = spec[h][i >> 1];
+                        f((i & 1) ? make_uint2(q.z, q.w) : make_uint2(q.x, q.y), h, i);
+                    }
+                const uint2 *src = sc.pcand + ((int64_t)l0 * NWV + h * ND + tid) * WCAP;
+                for (int i = SPEC; i < n; ++i) f(src[i], h, i);
+            }
+        };
+        if (greedy) {
+            // the first largest penalised logit (sample.c:130-132): every part's maxima are
+            // among its candidates unless a list overflowed; then the row is scanned
+            float bv = -INFINITY;
+            int bi = -1;
+            each_entry([&](uint2 e, int, int) { best_combine(bv, bi, key2f(e.x), (int)e.y); });
+            if (lane == 0) dl.offs[wv] = ovf;
+            __syncthreads();
+            int anyovf = 0;
+            for (int j = 0; j < ND / 64; ++j) anyovf |= dl.offs[j];
+            if (anyovf) {
+                bv = -INFINITY;
+                bi = -1;
+                row_visit<UNAL>(a, row, P, dl, [&](float w, int id) {
+                    if (w == w) best_combine(bv, bi, w, id);
+                });
+            }
+            block_best(bv, bi, dl);
+            if (tid == 0) record_greedy(row, P, bv, bi, dl.ct.maxl, x[0], st, a.out, a.diag);
+            return;
+        }
+        // only candidates above the row's bound are gathered: below it a list is incomplete
+        // (other parts may hold larger logits they did not keep), and the decision treats
+        // everything there as rejected
+        __syncthreads();
+        const uint32_t rej_row = dl.ct.rej;
+        int k0 = 0, k1 = 0;
+        each_entry([&](uint2 e, int h, int) {
+            if (e.x > rej_row) (h ? k1 : k0) += 1;
+        });
+        const int wincl = wave_scan(k0 + k1);
+        if (lane == 63) dl.exc[wv] = wincl;
         if (lane == 0) dl.offs[wv] = ovf;
         __syncthreads();
-        int anyovf = 0;
-        for (int j = 0; j < ND / 64; ++j) anyovf |= dl.offs[j];
-        if (anyovf) {
-            bv = -INFINITY;
-            bi = -1;
-            row_visit<UNAL>(a, row, P, dl, [&](float w, int id) {
-                if (w == w) best_combine(bv, bi, w, id);
+        int wbase = 0, total = 0, anyovf = 0;
+        for (int j = 0; j < ND / 64; ++j) {
+            if (j < wv) wbase += dl.exc[j];
+            total += dl.exc[j];
+            anyovf |= dl.offs[j];
+        }
+        t = dl.ct;
+        t.total = total;
+        t.cflag = anyovf;
+        const bool finite = isfinite(t.msc);
+        if (t.total <= FCAP && finite) {
+            int at = wbase + wincl - (k0 + k1);
+            each_entry([&](uint2 e, int, int) {
+                if (e.x > rej_row) {
+                    dl.keys[at] = e.x;
+                    dl.ids[at] = (int32_t)e.y;
+                    ++at;
+                }
             });
         }
-        block_best(bv, bi, dl);
-        if (tid == 0) record_greedy(row, P, bv, bi, dl.ct.maxl, x[0], st, a.out, a.diag);
-        return;
+        if (tid == 0) dl.ct = t;
+        __syncthreads();
+        status = !finite ? CF_INPUT
+                 : !(fabsf(t.msc) < CERT_MSC_MAX) || t.total > FCAP ? CF_MSC : DS_BLOCK;
     }
-    // only candidates above the row's bound are gathered: below it a list is incomplete
-    // (other parts may hold larger logits they did not keep), and the decision treats
-    // everything there as rejected
-    __syncthreads();
-    const uint32_t rej_row = dl.ct.rej;
-    int k0 = 0, k1 = 0;
-    each_entry([&](uint2 e, int h, int) {
-        if (e.x > rej_row) (h ? k1 : k0) += 1;
-    });
-    const int wincl = wave_scan(k0 + k1);
-    if (lane == 63) dl.exc[wv] = wincl;
-    if (lane == 0) dl.offs[wv] = ovf;
-    __syncthreads();
-    int wbase = 0, total = 0, anyovf = 0;
-    for (int j = 0; j < ND / 64; ++j) {
-        if (j < wv) wbase += dl.exc[j];
-        total += dl.exc[j];
-        anyovf |= dl.offs[j];
-    }
-    CertTotals t = dl.ct;
-    t.total = total;
-    t.cflag = anyovf;
-    const bool finite = isfinite(t.msc);
-    if (t.total <= FCAP && finite) {
-        int at = wbase + wincl - (k0 + k1);
-        each_entry([&](uint2 e, int, int) {
-            if (e.x > rej_row) {
-                dl.keys[at] = e.x;
-                dl.ids[at] = (int32_t)e.y;
-                ++at;
-            }
-        });
-    }
-    if (tid == 0) dl.ct = t;
-    __syncthreads();
-    int status = finite ? CF_MSC : CF_INPUT;
-    for (bool first = true; finite && fabsf(t.msc) < CERT_MSC_MAX && t.total <= FCAP;
-         first = false) {
+    // the gathered candidates, and once more with others (widen): one copy of this for rows of
+    // any number of parts (a copy in each branch made the kernel twice as large, and its
+    // instructions come from memory)
+    auto decide = [&]() __attribute__((always_inline)) {
         if (row_ksel(P) <= 64 && t.total <= WAVE_CAND) {
-            if (tid < 64) {
+            if (wv == 0) {
                 const int s = cert_row_wave(row, P, t, dl.keys, dl.ids, dl.srt, dl.dl.tab, st,
                                             a.out, a.diag, hist);
-                if (tid == 0) dl.dl.sh[7] = s;
+                if (lane == 0) dl.dl.sh[7] = s;
             }
             __syncthreads();
             status = dl.dl.sh[7];
@@ -1317,14 +1286,30 @@ __global__ void __launch_bounds__(ND) k_decide(PartArgs a, open::OpenArgs o) {
             status = cert_row_block<ND>(row, P, t, dl.keys, dl.ids, dl.srt, dl.dl, st, a.out,
                                         a.diag, hist);
         }
+    };
+    if (status == DS_BLOCK) {
+        decide();
         if (status == 0) return;
-        if (!WIDE || !first || !widen_pays(status, P, t)) break;
-        __syncthreads();
-        const bool more = widen<UNAL>(a, row, P, dl);
-        t = dl.ct;
-        if (!more) break;
     }
-    undecided(t, status);
+    if (WIDE && widen_pays(status, P, t)) {
+        __syncthreads();
+        if (widen<UNAL>(a, row, P, dl)) {
+            t = dl.ct;
+            decide();
+            if (status == 0) return;
+        }
+    }
+    if constexpr (OPEN) {
+        if (open::open_row(P, a.vocab) && isfinite(t.msc)) {
+            // left to k_open
+            if (tid == 0) {
+                o.s.ctl[row].reason = status;
+                o.s.queue[1 + add_dev(o.s.queue, 1)] = row;
+            }
+            return;
+        }
+    }
+    exact_row<UNAL>(a, row, P, t, dl, hist, status);
 }
 
 // The passes over the rows that k_decide queued (qs_open.h), a workgroup for each part of every
