@@ -1134,8 +1134,8 @@ int qs_batch_pick_ids(qs_batch *b, const float *d_logits, int64_t row_stride, in
 }
 
 int qs_batch_pick1_host(qs_batch *b, float *d_logits, const float *logits, int n_vocab,
-                        int32_t *d_out, int32_t *id) {
-    if (!b || !d_logits || !logits || !d_out || !id) return QS_EINVAL;
+                        int32_t *id) {
+    if (!b || !d_logits || !logits || !id) return QS_EINVAL;
     HIP_TRY(hipMemcpyAsync(d_logits, logits, sizeof(float) * (size_t)n_vocab,
                            hipMemcpyHostToDevice, b->stream), "logits to the device");
     return qs_batch_pick_ids(b, d_logits, n_vocab, 1, n_vocab, id);

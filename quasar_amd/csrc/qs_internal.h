@@ -42,10 +42,10 @@ int qs_debug_take_open_failure(void);     /* the same for qs_debug_fail_open_lau
 /* sample.h's pick of one row in one round trip: the host row copied to d_logits on the
  * batch's stream, then qs_batch_pick_ids: the kernels write the id (and the batch's error
  * flag) into pinned host memory, one wait.  QS_EAGAIN (the flag cleared) as
- * qs_batch_synchronize.  d_out is not used. */
+ * qs_batch_synchronize. */
 struct qs_batch;
 int qs_batch_pick1_host(struct qs_batch *b, float *d_logits, const float *logits, int n_vocab,
-                        int32_t *d_out, int32_t *id);
+                        int32_t *id);
 
 /* Thread-local error message used by qs_last_error(). */
 void qs_set_error(const char *fmt, ...);

@@ -27,7 +27,6 @@ struct quasar_sampler {
     int           vocab_cap;    /* widths the device buffers hold */
     int           ring_cap;     /* history capacity of the batch */
     float        *d_logits;
-    int32_t      *d_out;
     /* Host copy of the configuration, to re-apply when the batch is re-created and to
      * seed it when a config arrives before the first pick. */
     qs_row_param  prm;
@@ -84,10 +83,8 @@ quasar_sampler *quasar_sampler_new(void) {
 static void qs_release(quasar_sampler *s) {
     if (s->batch) qs_batch_free(s->batch);
     qs_device_free(s->d_logits);
-    qs_device_free(s->d_out);
     s->batch = NULL;
     s->d_logits = NULL;
-    s->d_out = NULL;
     s->vocab_cap = 0;
     s->ring_cap = 0;
 }
@@ -147,8 +144,7 @@ static int qs_ensure(quasar_sampler *s, int n_vocab) {
     int ring = s->prm.ring_cap;
     s->batch = qs_batch_new(1, n_vocab, ring);
     s->d_logits = (float *)qs_device_alloc(sizeof(float) * (size_t)n_vocab);
-    s->d_out = (int32_t *)qs_device_alloc(sizeof(int32_t));
-    if (!s->batch || !s->d_logits || !s->d_out) {
+    if (!s->batch || !s->d_logits) {
         qs_release(s);
         free(hist);
         return QS_ENOMEM;
@@ -177,11 +173,11 @@ int quasar_sampler_pick(quasar_sampler *s, const float *logits, int n_vocab) {
     int rc = qs_debug_take_failure() ? QS_ENOMEM : qs_ensure(s, n_vocab);
     int32_t id = -1;
     /* the row in, the pick, the id and the error flag out, one wait */
-    if (rc == 0) rc = qs_batch_pick1_host(s->batch, s->d_logits, logits, n_vocab, s->d_out, &id);
+    if (rc == 0) rc = qs_batch_pick1_host(s->batch, s->d_logits, logits, n_vocab, &id);
     /* A whole-window row that found no free scratch slot in time kept its state: pick it
      * again (a one-row batch has its own slot, so this is not expected). */
     for (int again = 0; rc == QS_EAGAIN && again < 3; ++again)
-        rc = qs_batch_pick1_host(s->batch, s->d_logits, logits, n_vocab, s->d_out, &id);
+        rc = qs_batch_pick1_host(s->batch, s->d_logits, logits, n_vocab, &id);
     if (rc == 0 && (id < 0 || id >= n_vocab)) rc = QS_EDEVICE;
     if (rc == 0) {
         host_record(s, id);

@@ -12,6 +12,7 @@
 #include "quasar_sampler.h"
 #include "../../oracle/orc_sampler.h"
 
+extern int stub_allocs;
 static int fails;
 #define CHECK(c) do { if (!(c)) { fprintf(stderr, "check failed: %s (line %d)\n", #c, __LINE__); fails++; } } while (0)
 
@@ -34,6 +35,9 @@ static void product(void) {
     int len = -1;
     quasar_sampler *s = quasar_sampler_new();
     CHECK(s != NULL);
+    fill(x, V);
+    (void)quasar_sampler_pick(s, x, V);
+    CHECK(stub_allocs == 1);                 /* the row of logits and nothing else */
     for (int round = 0; round < 3; round++) {
         quasar_sampler_config(s, 0.8f, 0.9f, 40 * round, 0.05f, 1.3f, 4 + round, 77u + round);
         for (int t = 0; t < 9; t++) {

@@ -36,8 +36,8 @@ int qs_batch_pick(qs_batch *b, const float *d_logits, int64_t row_stride, int n_
 }
 int qs_batch_synchronize(qs_batch *b) { (void)b; return QS_EDEVICE; }
 int qs_batch_pick1_host(struct qs_batch *b, float *d_logits, const float *logits, int n_vocab,
-                        int32_t *d_out, int32_t *id) {
-    (void)b; (void)d_logits; (void)logits; (void)n_vocab; (void)d_out; (void)id;
+                        int32_t *id) {
+    (void)b; (void)d_logits; (void)logits; (void)n_vocab; (void)id;
     return QS_EDEVICE;
 }
 int qs_batch_set_state(qs_batch *b, int row, uint64_t rng, const int32_t *hist, int n) {
@@ -48,7 +48,13 @@ int qs_batch_get_state(qs_batch *b, int row, uint64_t *rng, int32_t *hist, int c
     (void)b; (void)row; (void)rng; (void)hist; (void)cap; (void)len;
     return QS_EDEVICE;
 }
-void *qs_device_alloc(size_t bytes) { (void)bytes; NODEV("qs_device_alloc"); return NULL; }
+int stub_allocs;                       /* device allocations asked for */
+void *qs_device_alloc(size_t bytes) {
+    (void)bytes;
+    ++stub_allocs;
+    NODEV("qs_device_alloc");
+    return NULL;
+}
 void qs_device_free(void *p) { (void)p; }
 int qs_memcpy_h2d(void *d, const void *s, size_t n) { (void)d; (void)s; (void)n; return QS_EDEVICE; }
 int qs_memcpy_d2h(void *d, const void *s, size_t n) { (void)d; (void)s; (void)n; return QS_EDEVICE; }
