@@ -100,8 +100,9 @@ __device__ __forceinline__ int part_count(const PartArgs &a, int row, int j) {
 }
 
 // Visit the penalised logits at positions [from, to) of the row (from a multiple of 4; f(w, id)
-// on every thread's share; all threads): in blocks of XBM logits, each with its history bitmap in LDS, read XUP float4s per thread at
-// a time with every load issued before the first is used.  UNAL: rows at any alignment.
+// on every thread's share; all threads): in blocks of XBM logits, each with its history bitmap
+// in LDS, read XUP float4s per thread at a time with every load issued before the first is
+// used.  UNAL: rows at any alignment.
 template <bool UNAL, typename F>
 __device__ __forceinline__ void range_visit(const PartArgs &a, int row, const qs_row_param &P,
                                             DecLds &dl, int from, int to, F &&f) {

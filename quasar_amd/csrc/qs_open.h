@@ -16,11 +16,12 @@
 //     those bins and lists the (p, id) inside them.  The row's last part to finish finds
 //     the two positions in the lists.
 //
-// The decision kernel queues the rows it leaves undecided, and k_open takes the queue's.  In
-// picks of few rows the sums are taken by workgroups of the decision kernel past its row
-// decisions, beside them and for every row without a top-k (the chip is otherwise idle); in
-// larger picks that would hold up rows that need none, so a launch of its own (k_open_sum)
-// takes the queue's rows.  An empty queue costs a launch one load.
+// Both passes serve the rows that the decision kernel leaves undecided.  In picks of few rows
+// the sums are taken by workgroups of that kernel past its row decisions, beside them and for
+// every row without a top-k (the chip is otherwise idle).  In larger picks that would hold up
+// rows that need none: there the decision kernel queues its undecided rows, and a launch of its
+// own (k_open_sum), then k_open, take the queue's.  Rows that were decided cost these launches
+// one load a workgroup.
 //
 // Why it is the reference's result.  inv is proved to be the reference's float (inv_settled).
 // Every p is the reference's float.  Any order of adding n nonnegative binary64 numbers
@@ -29,13 +30,13 @@
 // by eps on both sides.  The order inside a list is exact, and a position counts only when
 // its p lies strictly between the least p above the list and the largest below it, so no
 // tie reaches across the list's ends.  Where inv is not settled (about one row in 1,000 at
-// 151,936 logits) the sum is taken again in id order; what is not proved (about one row in
-// 50,000, and rows of few values) takes full_row, as every such row did.
+// 151,936 logits) the sum is taken again in id order; what is not proved (3 of 60,000 rows of
+// N(0, 2) x 151,936, and rows of few values) takes full_row, as every such row did.
 // The histogram only chooses the bins: its error can cost a retry, never a result.
 //
-// Measured (8 rows of N(0, 2) x 151,936 logits, a pick with its ids on the host): 49 us
-// without cuts and 53 us at top-p 0.9, against 18.7 and 12.1 ms in one workgroup a row (with
-// the logits and lists requested only when first needed, 59 us without cuts).
+// Measured (8 rows of N(0, 2) x 151,936 logits, a pick with its ids on the host): 50 to 60 us
+// without cuts (by the logits: the ranked sub-bins hold up to 1,024 entries) and 54 us at top-p
+// 0.9, against 18.7 and 12.1 ms in one workgroup a row; the ids left on the device, 37 and 41.
 // Bounds: 8 rows x 151,936 logits are 4.9 MB, read from the last-level cache; the two
 // passes are instruction-bound (an expf a logit each) at about 300 workgroups, and the end
 // is a chain of block steps in one workgroup a row.

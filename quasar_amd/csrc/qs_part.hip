@@ -1,10 +1,10 @@
 // qs_part.hip - the streaming pick: one workgroup per part of a row, every logit read once,
 // then one workgroup per row for the decision.
 //
-// A pick of B rows of V logits (sample.c:111-179 per row) is two kernels (rows that are not
-// 16-byte aligned are read in whole 16-byte groups with the positions outside the row masked:
-// 48 rows of 100,003 logits, ids on the host, 90 us a pick through the split kernels' two
-// scalar passes, 59 us here):
+// A pick of B rows of V logits (sample.c:111-179 per row) is two kernels, and one or two more
+// where a row's top-k is off (qs_open.h).  Rows that are not 16-byte aligned are read in whole
+// 16-byte groups with the positions outside the row masked: 48 rows of 100,003 logits, ids on
+// the host, 90 us a pick through the split kernels' two scalar passes, 32 us here.
 //
 // k_part, B x P workgroups of 512 threads, P = ceil(V / 10240) parts per row (15 at
 // V = 151,936).  A workgroup holds its part in registers (five float4 per thread, the
@@ -963,9 +963,10 @@ __device__ __forceinline__ bool widen_pays(int why, const qs_row_param &P, const
 }
 
 // The row's bound is the largest part bound, and a part's bound is the least of its eight
-// wavefronts' maxima: now and then (about one row in 300 at top-k 40 and 10 parts) one lies so
-// high that fewer than top-k + 2 logits of the row exceed it, and such a row went to the exact
-// path, 170 us for its one workgroup.  Here the WIDEN parts with the largest bounds are read
+// wavefronts' maxima: now and then (at top-k 40, 26 of 6,000 rows of N(0, 2) x 100,000 logits, 4
+// of 6,000 x 151,936, none of 6,000 with one logit far ahead) one lies so high that fewer than
+// top-k + 2 logits of the row exceed it, and such a row went to the exact path, 170 us for its
+// one workgroup.  Here the WIDEN parts with the largest bounds are read
 // again for their logits in (r2, r1], r1 the row's bound and r2 the largest bound of the other
 // parts; with the other parts' candidates there (complete above r2) the row's bound becomes
 // r2.  All threads; dl.ct and the candidates are updated; false (dl.ct as it was) where the
@@ -1304,7 +1305,7 @@ __global__ void __launch_bounds__(ND) k_decide(PartArgs a, open::OpenArgs o) {
             // left to k_open
             if (tid == 0) {
                 o.s.ctl[row].reason = status;
-                o.s.queue[1 + add_dev(o.s.queue, 1)] = row;
+                if (!o.beside) o.s.queue[1 + add_dev(o.s.queue, 1)] = row;
             }
             return;
         }
@@ -1312,38 +1313,51 @@ __global__ void __launch_bounds__(ND) k_decide(PartArgs a, open::OpenArgs o) {
     exact_row<UNAL>(a, row, P, t, dl, hist, status);
 }
 
-// The passes over the rows that k_decide queued (qs_open.h), a workgroup for each part of every
-// row of the pick; those past the queue leave.  Neighbours take the same part of different
-// rows: their additions go to different histograms and counters.
-template <typename F>
-__device__ __forceinline__ void open_queue(const open::OpenArgs &o, F &&f) {
-    const int n = o.s.queue[0], i = blockIdx.x, part = n ? i / n : o.parts;
-    if (part < o.parts) f(o.s.queue[1 + i - part * n], part);
+// The passes over the rows that k_decide left (qs_open.h), a workgroup for each part of every
+// row of the pick.  Neighbours take the same part of different rows: their additions go to
+// different histograms and counters (a row's parts next to each other: 32 flat rows 80 us a
+// pick against 65).  The i-th workgroup's part of a queued row; those past the queue leave.
+__device__ __forceinline__ bool open_queued(const open::OpenArgs &o, int i, int &row, int &part) {
+    const int n = o.s.queue[0];
+    part = n ? i / n : o.parts;
+    if (part >= o.parts) return false;
+    row = o.s.queue[1 + i - part * n];
+    return true;
 }
 __global__ void __launch_bounds__(ND) k_open_sum(PartArgs a, open::OpenArgs o) {
     __shared__ open::OpenSumLds L;
-    open_queue(o, [&](int row, int part) { open::open_sum(a, o, row, part, L, c_tab_part); });
+    int row, part;
+    if (open_queued(o, blockIdx.x, row, part)) open::open_sum(a, o, row, part, L, c_tab_part);
 }
+static_assert((QS_PART_MAX_PARTS * QS_PART_LEN + open::OP - 1) / open::OP <= ND,
+              "a thread for each of a row's parts, where their records are read");
 template <bool UNAL>
 __global__ void __launch_bounds__(ND) k_open(PartArgs a, open::OpenArgs o) {
     constexpr size_t BYTES =
         sizeof(open::OpenLds) > sizeof(DecLds) ? sizeof(open::OpenLds) : sizeof(DecLds);
     __shared__ __align__(16) unsigned char lds[BYTES];
-    // a row decided although its sums were taken beside it: its histogram back to zero
-    if (o.beside && (int)blockIdx.x < a.n_rows && o.s.ctl[blockIdx.x].reason == 0)
-        for (int b = threadIdx.x; b < open::ONB; b += ND)
-            o.s.hist[(int64_t)blockIdx.x * open::ONB + b] = 0ull;
-    open_queue(o, [&](int row, int part) {
-        open::open_select<UNAL>(a, o, row, part, *(open::OpenLds *)lds, *(DecLds *)lds, c_tab_part);
-    });
+    int row, part;
+    if (o.beside) {                  // every row's sums are there: the queue's two loads saved
+        part = (int)blockIdx.x / a.n_rows;
+        row = (int)blockIdx.x - part * a.n_rows;
+        if (o.s.ctl[row].reason == 0) {               // decided: its histogram back to zero
+            if (part == 0)
+                for (int b = threadIdx.x; b < open::ONB; b += ND)
+                    o.s.hist[(int64_t)row * open::ONB + b] = 0ull;
+            return;
+        }
+    } else if (!open_queued(o, blockIdx.x, row, part)) {
+        return;
+    }
+    open::open_select<UNAL>(a, o, row, part, *(open::OpenLds *)lds, *(DecLds *)lds, c_tab_part);
 }
 
 // Up to this many workgroups of the first pass run beside the decisions (20 rows of 151,936);
 // past it they are a launch of their own, over the queue.  Rows without a top-k that the
 // certified decision covers, a pick beside / with the launch / with neither pass (an empty
-// launch is about 2.3 us): 8 rows 23 / - / 20.4 us, 17 rows 26.0 / 26.8 / -, 32 rows 30.2 / 26.7 /
-// 22.1, 60 rows 51 / 34 / 29: most of the first pass's workgroups wait for a place there.  Flat
-// rows lose the overlap: 17 rows 42 / 52 us, 32 rows 55 / 65, 60 rows 88 / 91.
+// launch is about 2.3 us): 8 rows 23 / - / 20.4 us, 17 rows 26.0 / 26.8 / -, 32 rows 30.2 / 25.7 /
+// 22.1, 60 rows 51 / 33 / 29: most of the first pass's workgroups wait for a place there.  Flat
+// rows lose the overlap: 17 rows 42 / 52 us, 32 rows 55 / 64, 60 rows 88 / 91.
 constexpr unsigned OPEN_BESIDE = 768;
 
 }  // namespace
@@ -1441,10 +1455,11 @@ int qs_part_launch(const float *logits, int64_t row_stride, int n_rows, int n_vo
             oa.beside = np <= OPEN_BESIDE;
             if (oa.beside) beside = np;
         }
-        // The widening costs every decision about 0.5 us (its registers and code: one row 15.9
-        // against 16.3 us a pick, 32 rows 31.5 against 32.2) and saves a row that needs it 170,
-        // about one in 300 (unaligned 48-row batches: one in seven held such a row), so it
-        // pays from a few rows on.
+        // The widening costs every pick about 0.3 us (its code: 4 aligned rows 16.9 us a pick
+        // without, 5 rows 17.2 with) and saves a row that needs it 170.  At 151,936 logits one
+        // flat row in 1,500 does: 0.1 us a row, so it pays from about four rows on.  At 100,000
+        // it is one in 230 and would pay for one row too; there too the smallest aligned picks
+        // keep their usual time.  (Unaligned picks have no decision without it.)
         const bool wide = n_rows > 4;
         auto *k = unal   ? (open ? k_decide<true, true, true> : k_decide<false, true, true>)
                   : wide ? (open ? k_decide<true, false, true> : k_decide<false, false, true>)
