@@ -18,8 +18,8 @@
  * sampler's first pass in its epilogue, and the pick of every row from it.
  *
  * Return codes of the extension functions: 0 on success, QS_EINVAL for bad arguments,
- * QS_ENOMEM when device memory cannot be allocated, QS_EAGAIN (qs_batch_synchronize only)
- * when rows must be picked again, QS_EDEVICE for any other HIP failure; qs_last_error()
+ * QS_ENOMEM when device memory cannot be allocated, QS_EAGAIN (qs_batch_synchronize and
+ * qs_batch_pick_ids) when rows must be picked again, QS_EDEVICE for any other HIP failure; qs_last_error()
  * describes the last failure on the calling thread.
  */
 #ifndef QUASAR_SAMPLER_H
@@ -83,8 +83,9 @@ int qs_debug_fail_picks(int n);
 #define QS_EINVAL  (-22)
 #define QS_ENOMEM  (-12)
 #define QS_EDEVICE (-5)
-#define QS_EAGAIN  (-11)   /* qs_batch_synchronize: some rows could not take a whole-window
-                              scratch slot in time; they returned -3 and kept their state */
+#define QS_EAGAIN  (-11)   /* qs_batch_synchronize and qs_batch_pick_ids: some rows could not
+                              take a whole-window scratch slot in time; they returned -3 and
+                              kept their state */
 
 typedef struct qs_batch qs_batch;
 
@@ -179,7 +180,8 @@ int qs_batch_pick_ids(qs_batch *b, const float *d_logits, int64_t row_stride, in
  * every logit read once and the row decided from LDS (16-byte aligned rows, a vocabulary
  * and a row stride that are multiples of 4, vocabulary up to 262,144).  STREAM: two
  * kernels, every logit read once by workgroups that each take a part of a row, then one
- * decision workgroup per row (the same alignment, vocabulary up to 655,360).  SPLIT:
+ * decision workgroup per row, and one or two more for rows whose top-k is off (the same
+ * alignment, vocabulary up to 655,360).  SPLIT:
  * three kernels per pick, the logits streamed twice (any layout).  A mode that does not
  * support a pick returns QS_EINVAL.  The results are identical. */
 enum { QS_MODE_AUTO = 0, QS_MODE_SPLIT = 1, QS_MODE_STREAM = 2, QS_MODE_ROW = 3 };
